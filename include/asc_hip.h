@@ -98,8 +98,8 @@ int32_t asc_module_launch(void* function, uint32_t grid, uint32_t block,
 /* A launch of one kernel of a prebuilt code object whose argument is a single
  * struct: the kernel's symbol, its grid and block, and the struct's bytes as the
  * argument blob asc_module_launch takes.  asc_flash_attention_plan,
- * asc_matmul_plan and asc_matmul_i8_plan fill it with exactly the launch their
- * library entry points make.  No counterpart in the reference, whose compiler
+ * asc_matmul_dispatch and asc_matmul_i8_dispatch fill it with exactly the launch
+ * their library entry points make.  No counterpart in the reference, whose compiler
  * fixes the launch inside the kernel binary. */
 typedef struct asc_launch_plan {
   char kernel[64];   /* NUL-terminated symbol; empty when there is nothing to launch */
@@ -326,8 +326,9 @@ int32_t asc_matmul_chained_noalloc(int32_t in_dtype, int32_t out_dtype,
                                    const void* a, const void* b, void* c,
                                    int64_t M, int64_t N, int64_t K,
                                    asc_stream_t stream);
-/* The launch asc_matmul_bias_act makes with these arguments (asc_matmul(...,
- * relu) is act = relu, bias NULL), as a kernel of the code object
+/* A launch of asc_matmul_bias_act's product (asc_matmul(..., relu) is act = relu,
+ * bias NULL) by the kernel of its operands' type on 256x256 tiles (fp32: 16x16
+ * blocks or 64x64 tiles), as a kernel of the code object
  * pyasc_amd/lib/co/asc2_matmul.hsaco (asc_launch_plan_t; the blob is the
  * kernel's argument struct).  Same checks and errors. */
 int32_t asc_matmul_plan(int32_t in_dtype, int32_t out_dtype, const void* a,
@@ -335,6 +336,15 @@ int32_t asc_matmul_plan(int32_t in_dtype, int32_t out_dtype, const void* a,
                         int64_t N, int64_t K, int64_t lda, int64_t ldb,
                         int64_t ldc, int32_t act, float alpha,
                         asc_launch_plan_t* plan);
+/* The launch asc_matmul_bias_act makes with these arguments (asc_matmul(...,
+ * relu) is act = relu, bias NULL): asc_matmul_plan's where its kernel is the
+ * fastest for the shape, else one of the tile kernels asc2_mm_tile_* of the same
+ * code object.  Same arguments, checks and errors as asc_matmul_plan. */
+int32_t asc_matmul_dispatch(int32_t in_dtype, int32_t out_dtype, const void* a,
+                            const void* b, void* c, const float* bias,
+                            int64_t M, int64_t N, int64_t K, int64_t lda,
+                            int64_t ldb, int64_t ldc, int32_t act, float alpha,
+                            asc_launch_plan_t* plan);
 
 /* ---- int8 matmul with per-channel dequant -----------------------------------
  * asc1 matmul_kernel(a, b, c, tiling, workspace, quant_vector) with
@@ -356,13 +366,20 @@ int32_t asc_matmul_i8_dequant_f16(const int8_t* a, const int8_t* b,
                                   const float* scale, void* c, int64_t M,
                                   int64_t N, int64_t K, int32_t trunc19,
                                   asc_stream_t stream);
-/* The launch asc_matmul_i8_i32 (dequant 0; scale and trunc19 ignored) or
- * asc_matmul_i8_dequant_f16 (dequant 1) makes, as a kernel of the code object
- * pyasc_amd/lib/co/asc2_matmul_i8.hsaco.  Same checks and errors. */
+/* A launch of asc_matmul_i8_i32's product (dequant 0; scale and trunc19 ignored)
+ * or asc_matmul_i8_dequant_f16's (dequant 1) on 256x256 tiles, as a kernel of the
+ * code object pyasc_amd/lib/co/asc2_matmul_i8.hsaco.  Same checks and errors. */
 int32_t asc_matmul_i8_plan(const int8_t* a, const int8_t* b, const float* scale,
                            void* c, int64_t M, int64_t N, int64_t K,
                            int32_t dequant, int32_t trunc19,
                            asc_launch_plan_t* plan);
+/* The launch the two entries make: asc_matmul_i8_plan's where its kernel is the
+ * fastest for the shape, else one of the tile kernels asc2_i8_tile_* of the same
+ * code object.  Same arguments, checks and errors as asc_matmul_i8_plan. */
+int32_t asc_matmul_i8_dispatch(const int8_t* a, const int8_t* b,
+                               const float* scale, void* c, int64_t M,
+                               int64_t N, int64_t K, int32_t dequant,
+                               int32_t trunc19, asc_launch_plan_t* plan);
 
 /* ---- flash-attention forward ---------------------------------------------------
  * No reference function exists (the reference has no attention kernel); this

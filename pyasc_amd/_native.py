@@ -85,6 +85,10 @@ SIGNATURES = {
                                  ctypes.POINTER(LaunchPlan)],
     "asc_matmul_plan": [_c_i32, _c_i32, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i32,
                         _c_f32, ctypes.POINTER(LaunchPlan)],
+    "asc_matmul_dispatch": [_c_i32, _c_i32, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+                            _c_i32, _c_f32, ctypes.POINTER(LaunchPlan)],
+    "asc_matmul_i8_dispatch": [_c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i32, _c_i32,
+                               ctypes.POINTER(LaunchPlan)],
     "asc_matmul_i8_plan": [_c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i32, _c_i32, ctypes.POINTER(LaunchPlan)],
     "asc_unary_f32": [_c_i32, _c_p, _c_p, _c_i64, _c_p],
     "asc_binary": [_c_i32, _c_i32, _c_p, _c_p, _c_p, _c_i64, _c_i32, _c_f64, _c_i64, _c_p],

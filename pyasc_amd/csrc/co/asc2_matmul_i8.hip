@@ -4,8 +4,11 @@
 // loaded with hipModuleLoad by the asc2 launch path (pyasc_amd/asc/runtime/module.py)
 // as the reference loads the binary its compiler produced
 // (python/asc/runtime/jit.py:158-186).  asc2_i8_{fast,checked}_{i32,f16} take one
-// asc::i8::I8Args by value; asc_matmul_i8_plan fills it, with the grid and block,
-// exactly as the library's asc_matmul_i8_* entries launch them.
+// asc::i8::I8Args by value, asc2_i8_tile_<tile> one asc::gemm::TileArgs;
+// asc_matmul_i8_dispatch fills it, with the grid and block, exactly as the library's
+// asc_matmul_i8_* entries launch them.
 #include "matmul_i8_kernels.h"
+#include "matmul_tile.h"
 
 ASC_I8_KERNELS(extern "C", asc2_i8_)
+ASC_TILE_KERNELS_MFMA(ASC_TILE_DEFINE, extern "C", asc2_i8_tile_, asc::tile::TrI8)

@@ -3,6 +3,9 @@
 // entry points and the launch plan the asc2 code-object path replays.  The device
 // code is matmul_i8_kernels.h.
 #include "matmul_i8_kernels.h"
+#include "matmul_tile.h"
+
+ASC_TILE_KERNELS_I8(ASC_TILE_DECLARE, , asc_tile_)
 
 namespace {
 
@@ -59,11 +62,47 @@ int32_t make_launch(const int8_t* a, const int8_t* b, const float* scale, void* 
   return ASC_OK;
 }
 
+// ---- tile kernels (matmul_tile.h)
+using asc::tile::TileLaunch;
+using TileFn = void (*)(asc::gemm::TileArgs);
+const TileFn kTileI8[asc::tile::kNumDma + asc::tile::kNumAny] = ASC_TILE_TABLE_MFMA(asc_tile_i8_);
+
+// The tile launch that takes the call of a checked, non-empty I8Launch, or T.index < 0 when
+// L's own kernel runs it: K == 0, or the tile-aligned loop on its own 256x256 tiles.
+void make_tile(int mode, const I8Launch& L, TileLaunch& T) {
+  T = TileLaunch{};
+  const I8Args& g = L.p;
+  if (g.K == 0) return;
+  const bool dma = asc::tile::dma_takes(g.a, g.b, g.N, g.K, g.K, g.N, 1);
+  asc::tile::choose_mfma(1, dma, g.M, g.N, g.K, T);
+  if (T.index == asc::tile::kD256x256 && L.kernel < 2) T.index = -1;
+  asc::gemm::TileArgs& p = T.p;
+  p.a = g.a;
+  p.b = g.b;
+  p.c = g.c;
+  p.vec = mode == 1 ? g.scale : nullptr;
+  p.lda = g.K;
+  p.ldb = g.N;
+  p.ldc = g.N;
+  p.M = g.M;
+  p.N = g.N;
+  p.K = g.K;
+  p.out = mode == 1 ? asc::gemm::kTileOutF16 : asc::gemm::kTileOutI32;
+  p.trunc19 = g.trunc19;
+}
+
 int32_t run(const int8_t* a, const int8_t* b, const float* scale, void* c, int64_t M, int64_t N, int64_t K,
             int32_t trunc19, int mode, asc_stream_t stream, const char* who) {
   I8Launch L;
   const int32_t rc = make_launch(a, b, scale, c, M, N, K, trunc19, mode, who, L);
   if (rc != ASC_OK || L.blocks == 0) return rc;
+  TileLaunch T;
+  make_tile(mode, L, T);
+  if (T.index >= 0) {
+    hipLaunchKernelGGL(kTileI8[T.index], dim3(static_cast<uint32_t>(T.blocks)), dim3(T.threads), 0,
+                       static_cast<hipStream_t>(stream), T.p);
+    return asc::check_launch(who);
+  }
   decltype(&gemm_i8_fast_i32) const kernels[4] = {gemm_i8_fast_i32, gemm_i8_fast_f16, gemm_i8_checked_i32,
                                                   gemm_i8_checked_f16};
   hipLaunchKernelGGL(kernels[L.kernel], dim3(static_cast<uint32_t>(L.blocks)), dim3(L.threads), 0,
@@ -83,20 +122,57 @@ extern "C" int32_t asc_matmul_i8_dequant_f16(const int8_t* a, const int8_t* b, c
   return run(a, b, scale, c, M, N, K, trunc19, 1, stream, "asc_matmul_i8_dequant_f16");
 }
 
-extern "C" int32_t asc_matmul_i8_plan(const int8_t* a, const int8_t* b, const float* scale, void* c, int64_t M,
-                                      int64_t N, int64_t K, int32_t dequant, int32_t trunc19,
-                                      asc_launch_plan_t* plan) {
-  ASC_REQUIRE(plan, ASC_ERR_INVALID_ARG, "asc_matmul_i8_plan: null plan");
-  *plan = asc_launch_plan_t{};
-  I8Launch L;
-  const int32_t rc = make_launch(a, b, dequant ? scale : nullptr, c, M, N, K, dequant ? trunc19 : 0, dequant ? 1 : 0,
-                                 dequant ? "asc_matmul_i8_dequant_f16" : "asc_matmul_i8_i32", L);
-  if (rc != ASC_OK || L.blocks == 0) return rc;
+namespace {
+
+// `L`'s own kernel as a plan.
+void fill_plan(const I8Launch& L, asc_launch_plan_t* plan) {
   static_assert(sizeof(I8Args) <= sizeof(plan->args), "argument blob");
   __builtin_strncpy(plan->kernel, kI8Kernels[L.kernel], sizeof(plan->kernel) - 1);
   plan->grid = static_cast<uint32_t>(L.blocks);
   plan->block = static_cast<uint32_t>(L.threads);
   plan->args_size = sizeof(I8Args);
   __builtin_memcpy(plan->args, &L.p, sizeof(I8Args));
+}
+
+int32_t checked_launch(const int8_t* a, const int8_t* b, const float* scale, void* c, int64_t M, int64_t N, int64_t K,
+                       int32_t dequant, int32_t trunc19, I8Launch& L) {
+  return make_launch(a, b, dequant ? scale : nullptr, c, M, N, K, dequant ? trunc19 : 0, dequant ? 1 : 0,
+                     dequant ? "asc_matmul_i8_dequant_f16" : "asc_matmul_i8_i32", L);
+}
+
+}  // namespace
+
+extern "C" int32_t asc_matmul_i8_plan(const int8_t* a, const int8_t* b, const float* scale, void* c, int64_t M,
+                                      int64_t N, int64_t K, int32_t dequant, int32_t trunc19,
+                                      asc_launch_plan_t* plan) {
+  ASC_REQUIRE(plan, ASC_ERR_INVALID_ARG, "asc_matmul_i8_plan: null plan");
+  *plan = asc_launch_plan_t{};
+  I8Launch L;
+  const int32_t rc = checked_launch(a, b, scale, c, M, N, K, dequant, trunc19, L);
+  if (rc != ASC_OK || L.blocks == 0) return rc;
+  fill_plan(L, plan);
+  return ASC_OK;
+}
+
+extern "C" int32_t asc_matmul_i8_dispatch(const int8_t* a, const int8_t* b, const float* scale, void* c, int64_t M,
+                                          int64_t N, int64_t K, int32_t dequant, int32_t trunc19,
+                                          asc_launch_plan_t* plan) {
+  ASC_REQUIRE(plan, ASC_ERR_INVALID_ARG, "asc_matmul_i8_dispatch: null plan");
+  *plan = asc_launch_plan_t{};
+  I8Launch L;
+  const int32_t rc = checked_launch(a, b, scale, c, M, N, K, dequant, trunc19, L);
+  if (rc != ASC_OK || L.blocks == 0) return rc;
+  TileLaunch T;
+  make_tile(dequant ? 1 : 0, L, T);
+  if (T.index < 0) {
+    fill_plan(L, plan);
+    return ASC_OK;
+  }
+  static_assert(sizeof(T.p) <= sizeof(plan->args), "argument blob");
+  __builtin_snprintf(plan->kernel, sizeof(plan->kernel), "asc2_i8_tile_%s", T.name);
+  plan->grid = static_cast<uint32_t>(T.blocks);
+  plan->block = static_cast<uint32_t>(T.threads);
+  plan->args_size = sizeof(T.p);
+  __builtin_memcpy(plan->args, &T.p, sizeof(T.p));
   return ASC_OK;
 }

@@ -390,11 +390,20 @@ def matmul_chained(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, workspace:
 
 def matmul_plan(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, relu: bool = False,
                 bias: Optional[torch.Tensor] = None, leaky_alpha: Optional[float] = None) -> "_native.LaunchPlan":
-    """The launch matmul(...) makes, as a kernel of the asc2_matmul code object with its
-    grid, block and argument blob (asc_matmul_plan); plan.grid == 0 when there is nothing
-    to launch.  Same checks and errors as matmul."""
+    """A launch of matmul(...)'s product by the kernel of its type on 256x256 tiles (fp32: 16x16
+    blocks or 64x64 tiles), as a kernel of the asc2_matmul code object with its grid, block and
+    argument blob (asc_matmul_plan); plan.grid == 0 when there is nothing to launch.  Same
+    checks and errors as matmul."""
     plan = _native.LaunchPlan()
     _native.call("asc_matmul_plan", *_matmul_args(a, b, c, relu, bias, leaky_alpha), ctypes.byref(plan))
+    return plan
+
+
+def matmul_dispatch(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, relu: bool = False,
+                    bias: Optional[torch.Tensor] = None, leaky_alpha: Optional[float] = None) -> "_native.LaunchPlan":
+    """The launch matmul(...) makes (asc_matmul_dispatch), in matmul_plan's form."""
+    plan = _native.LaunchPlan()
+    _native.call("asc_matmul_dispatch", *_matmul_args(a, b, c, relu, bias, leaky_alpha), ctypes.byref(plan))
     return plan
 
 
@@ -437,10 +446,19 @@ def matmul_i8(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, scale: Optional
 
 def matmul_i8_plan(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, scale: Optional[torch.Tensor] = None,
                    trunc19: bool = False) -> "_native.LaunchPlan":
-    """The launch matmul_i8(...) makes, as a kernel of the asc2_matmul_i8 code object with
-    its grid, block and argument blob (asc_matmul_i8_plan).  Same checks as matmul_i8."""
+    """A launch of matmul_i8(...)'s product on 256x256 tiles, as a kernel of the asc2_matmul_i8
+    code object with its grid, block and argument blob (asc_matmul_i8_plan).  Same checks as
+    matmul_i8."""
     plan = _native.LaunchPlan()
     _native.call("asc_matmul_i8_plan", *_matmul_i8_args(a, b, c, scale, trunc19), ctypes.byref(plan))
+    return plan
+
+
+def matmul_i8_dispatch(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, scale: Optional[torch.Tensor] = None,
+                       trunc19: bool = False) -> "_native.LaunchPlan":
+    """The launch matmul_i8(...) makes (asc_matmul_i8_dispatch), in matmul_i8_plan's form."""
+    plan = _native.LaunchPlan()
+    _native.call("asc_matmul_i8_dispatch", *_matmul_i8_args(a, b, c, scale, trunc19), ctypes.byref(plan))
     return plan
 
 

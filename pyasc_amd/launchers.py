@@ -330,14 +330,14 @@ def _merge_full(rects: List[Tuple[int, int, int, int]], M: int, N: int) -> List[
 
 
 # The asc2 matmul bodies take the matmul they launch: kernels.matmul (the library's
-# asc_matmul) or, for a code-object launch, the same call replayed from asc_matmul_plan
+# asc_matmul) or, for a code-object launch, the same call replayed from asc_matmul_dispatch
 # through the asc2_matmul code object.  Either way the same kernels run with the same
 # arguments.
 
 def _matmul_through(functions, stream):
     """kernels.matmul's call form, launched through the asc2_matmul code object."""
     def mm(a, b, c, relu=False, stream=stream, bias=None, leaky_alpha=None):
-        module.launch_plan(functions, kernels.matmul_plan(a, b, c, relu=relu, bias=bias, leaky_alpha=leaky_alpha),
+        module.launch_plan(functions, kernels.matmul_dispatch(a, b, c, relu=relu, bias=bias, leaky_alpha=leaky_alpha),
                            stream)
     return mm
 
@@ -398,10 +398,17 @@ def _chained_body(call: KernelCall, mm, chained=None) -> None:
         t.record_stream(torch.cuda.ExternalStream(call.stream, device=a.device))
 
 
+# The tile kernels of csrc/matmul_tile.h: fp16 / bf16 / int8, and fp32.
+TILE_VARIANTS = ("256x256", "128x256", "192x128", "128x128", "64x64", "64x64k2", "32x64", "32x32", "any_256x256",
+                 "any_128x128", "any_64x64", "any_32x32")
+TILE_VARIANTS_F32 = ("128x128", "64x64", "32x32", "any_128x128", "any_64x64", "any_32x32")
+
 # The kernels of the asc2_matmul code object (csrc/co/asc2_matmul.hip).
 MATMUL_CO_FUNCTIONS = tuple(
     f"asc2_mm_{kind}_{out}" for out in ("f32", "f16", "bf16")
-    for kind in ("mfma_bf16_fast", "mfma_bf16_checked", "mfma_f16_fast", "mfma_f16_checked", "f32_mfma", "f32_fma"))
+    for kind in ("mfma_bf16_fast", "mfma_bf16_checked", "mfma_f16_fast", "mfma_f16_checked", "f32_mfma", "f32_fma")) + \
+    tuple(f"asc2_mm_tile_{dtype}_{tile}" for dtype in ("bf16", "f16") for tile in TILE_VARIANTS) + \
+    tuple(f"asc2_mm_tile_f32_{tile}" for tile in TILE_VARIANTS_F32)
 
 
 def _matmul_code_object(body) -> module.CodeObject:
@@ -454,13 +461,14 @@ def _trunc_scale(call: KernelCall) -> bool:
 
 
 # The kernels of the asc2_matmul_i8 code object (csrc/co/asc2_matmul_i8.hip).
-MATMUL_I8_CO_FUNCTIONS = tuple(f"asc2_i8_{path}_{out}" for path in ("fast", "checked") for out in ("i32", "f16"))
+MATMUL_I8_CO_FUNCTIONS = tuple(f"asc2_i8_{path}_{out}" for path in ("fast", "checked") for out in ("i32", "f16")) + \
+    tuple(f"asc2_i8_tile_{tile}" for tile in TILE_VARIANTS)
 
 
 def _i8_code_object(launch) -> module.CodeObject:
     def run(call: KernelCall, functions) -> None:
         def mm8(a, b, c, scale=None, trunc19=False):
-            module.launch_plan(functions, kernels.matmul_i8_plan(a, b, c, scale=scale, trunc19=trunc19),
+            module.launch_plan(functions, kernels.matmul_i8_dispatch(a, b, c, scale=scale, trunc19=trunc19),
                                call.stream)
         launch(call, mm8)
     return module.CodeObject("asc2_matmul_i8", MATMUL_I8_CO_FUNCTIONS, run, "pyasc_amd/csrc/co/asc2_matmul_i8.hip")

@@ -1,0 +1,120 @@
+"""asc_matmul_dispatch and asc_matmul_i8_dispatch without a GPU: the launch the matmul entries
+make.  Every dispatched launch covers C with whole tiles, fits one launch, carries the call's
+arguments, uses the direct-to-LDS tiles only on operands made of 16-byte chunks, and fails
+exactly where the plan of the 256x256-tile kernels fails.  Over many shapes the choice reaches
+every tile kernel of the code objects."""
+import ctypes
+import random
+import re
+import struct
+
+from hypothesis import given, settings, strategies as st
+
+from pyasc_amd import _native
+from pyasc_amd.launchers import MATMUL_CO_FUNCTIONS, MATMUL_I8_CO_FUNCTIONS
+
+A, B, C, BIAS = 0x100000, 0x200000, 0x300000, 0x400000  # 16-byte aligned stand-ins, never dereferenced
+F32, F16, BF16 = _native.DT_FLOAT32, _native.DT_FLOAT16, _native.DT_BFLOAT16
+ES = {F32: 4, F16: 2, BF16: 2}
+# TileArgs: a, b, c, vec, lda, ldb, ldc, M, N, K, tiles_m, tiles_n, out, act, alpha, trunc19, reserved
+TILE_ARGS = struct.Struct("<QQQQqqqiiiiiiifii")
+
+
+def lib():
+    return _native.load_library()
+
+
+def mm(fn, in_dt, out_dt, M, N, K, lda, ldb, ldc, a=A, act=0, alpha=0.0, bias=0):
+    p = _native.LaunchPlan()
+    return getattr(lib(), fn)(in_dt, out_dt, a, B, C, bias, M, N, K, lda, ldb, ldc, act, alpha, ctypes.byref(p)), p
+
+
+def tile_of(name):
+    bm, bn = re.search(r"(\d+)x(\d+)(?:k2)?$", name).groups()
+    return int(bm), int(bn)
+
+
+def check_tile(p, a, M, N, K, lda, ldb, ldc, es, offset):
+    bm, bn = tile_of(p.kernel.decode())
+    args = TILE_ARGS.unpack(p.blob())
+    assert p.args_size == TILE_ARGS.size and args[0] == a and args[4:10] == (lda, ldb, ldc, M, N, K)
+    tm, tn = -(-M // bm), -(-N // bn)
+    assert args[10:12] == (tm, tn) and p.grid == tm * tn and p.grid * p.block < 2 ** 32
+    aligned = offset % 16 == 0 and all(v * es % 16 == 0 for v in (lda, ldb, N, K))
+    small = 256 * lda * es + K * es < 2 ** 31 - 2 ** 20 and 128 * ldb * es < 2 ** 31 - 2 ** 20
+    assert ("_any_" not in p.kernel.decode()) == (aligned and small)
+
+
+@settings(max_examples=600, deadline=None)
+@given(in_dt=st.sampled_from([F32, F16, BF16]), out_dt=st.sampled_from([F32, F16, BF16]), M=st.integers(0, 20000),
+       N=st.integers(0, 20000), K=st.integers(0, 20000), unit=st.sampled_from([1, 8, 256]), pad=st.integers(0, 64),
+       a_off=st.sampled_from([0, 2, 16]))
+def test_matmul_dispatch_properties(in_dt, out_dt, M, N, K, unit, pad, a_off):
+    M, N, K = (v // unit * unit for v in (M, N, K))
+    args = (in_dt, out_dt, M, N, K, K + pad, N, N)
+    rc, p = mm("asc_matmul_dispatch", *args, a=A + a_off)
+    rc0, p0 = mm("asc_matmul_plan", *args, a=A + a_off)
+    assert rc == rc0
+    if rc != 0 or M == 0 or N == 0:
+        assert p.grid == 0
+        return
+    name = p.kernel.decode()
+    assert name in MATMUL_CO_FUNCTIONS
+    if "_tile_" not in name:  # the plan's own kernel, argument for argument
+        assert (name, p.grid, p.block, p.blob()) == (p0.kernel.decode(), p0.grid, p0.block, p0.blob())
+        assert K == 0 or "_fast_" in name or "f32_mfma" in name
+        return
+    assert K > 0 and f"_tile_{({F32: 'f32', F16: 'f16', BF16: 'bf16'}[in_dt])}_" in name
+    check_tile(p, A + a_off, M, N, K, K + pad, N, N, ES[in_dt], a_off)
+    assert TILE_ARGS.unpack(p.blob())[12] == {F32: 0, F16: 1, BF16: 2}[out_dt]
+
+
+@settings(max_examples=400, deadline=None)
+@given(M=st.integers(0, 30000), N=st.integers(0, 30000), K=st.integers(0, 1 << 17), unit=st.sampled_from([1, 16, 256]),
+       dequant=st.booleans(), a_off=st.sampled_from([0, 1, 16]))
+def test_int8_dispatch_properties(M, N, K, unit, dequant, a_off):
+    M, N, K = (v // unit * unit for v in (M, N, K))
+    p, p0 = _native.LaunchPlan(), _native.LaunchPlan()
+    args = (A + a_off, B, BIAS, C, M, N, K, int(dequant), 1)
+    assert lib().asc_matmul_i8_dispatch(*args, ctypes.byref(p)) == 0
+    assert lib().asc_matmul_i8_plan(*args, ctypes.byref(p0)) == 0
+    if M == 0 or N == 0:
+        assert p.grid == 0
+        return
+    name = p.kernel.decode()
+    assert name in MATMUL_I8_CO_FUNCTIONS
+    if "_tile_" not in name:
+        assert (name, p.grid, p.block, p.blob()) == (p0.kernel.decode(), p0.grid, p0.block, p0.blob())
+        assert K == 0 or "_fast_" in name
+        return
+    check_tile(p, A + a_off, M, N, K, K, N, N, 1, a_off)
+    out = TILE_ARGS.unpack(p.blob())
+    assert (out[3], out[12], out[15]) == ((BIAS, 1, 1) if dequant else (0, 3, 0))
+
+
+def test_dispatch_errors_match_the_plans():
+    for args in ((F16, F16, 0, 0, 0, 0, -1, 8, 8, 8, 8, 8, 0, 0.0), (F16, F16, A, B, C, 0, 8, 8, 8, 4, 8, 8, 0, 0.0),
+                 (F16, F16, 0, 0, C, 0, 8, 8, 8, 8, 8, 8, 0, 0.0), (3, F16, A, B, C, 0, 8, 8, 8, 8, 8, 8, 0, 0.0),
+                 (F16, F16, A, B, C, 0, 8, 8, 8, 8, 8, 8, 3, 0.0),
+                 (F16, F16, A, B, C, 0, 1 << 29, 1 << 29, 32, 32, 1 << 29, 1 << 29, 0, 0.0)):
+        p = _native.LaunchPlan()
+        assert lib().asc_matmul_dispatch(*args, ctypes.byref(p)) == lib().asc_matmul_plan(*args, ctypes.byref(p)) != 0
+    p = _native.LaunchPlan()
+    assert lib().asc_matmul_i8_dispatch(A, B, 0, C, 8, 8, 8, 1, 0, ctypes.byref(p)) == _native.ERR_INVALID_ARG
+    assert lib().asc_matmul_i8_dispatch(A, B, 0, C, 8, 8, (1 << 17) + 1, 0, 0, ctypes.byref(p)) == \
+        _native.ERR_UNSUPPORTED
+
+
+def test_every_tile_kernel_is_reached():
+    rng = random.Random(5)
+    seen = set()
+    for _ in range(6000):
+        M, N, K = (int(2 ** rng.uniform(0, 13.5)) for _ in range(3))
+        if rng.random() < 0.7:
+            N, K = max(16, N // 16 * 16), max(16, K // 16 * 16)
+        for dt in (F32, F16, BF16):
+            seen.add(mm("asc_matmul_dispatch", dt, F32, M, N, K, K, N, N)[1].kernel.decode())
+        p = _native.LaunchPlan()
+        assert lib().asc_matmul_i8_dispatch(A, B, BIAS, C, M, N, K, 1, 0, ctypes.byref(p)) == 0
+        seen.add(p.kernel.decode())
+    assert {n for n in MATMUL_CO_FUNCTIONS + MATMUL_I8_CO_FUNCTIONS if "_tile_" in n} <= seen
