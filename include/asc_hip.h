@@ -248,6 +248,19 @@ int32_t asc_softmax_plan(int32_t dtype, int32_t fused, const void* x,
 int32_t asc_reduce_f32(int32_t op, const float* x, float* out, int64_t rows,
                        int64_t cols, int32_t dim, int64_t out_count,
                        asc_stream_t stream);
+/* asc_reduce_f32 with a workspace for partial results (no counterpart in the
+ * reference): reductions with few results over many elements are split over the
+ * whole chip and combined by a second launch, in a fixed order.
+ * asc_reduce_f32_workspace gives the bytes it needs (at most 65536; 0: it would not
+ * be used).
+ * The workspace (NULL: as asc_reduce_f32) must be 4-byte aligned, hold that many
+ * bytes and not overlap x or out; both launches run in order on `stream`, so it
+ * may be reused once they have run. */
+int32_t asc_reduce_f32_workspace(int64_t rows, int64_t cols, int32_t dim);
+int32_t asc_reduce_f32_ws(int32_t op, const float* x, float* out, int64_t rows,
+                          int64_t cols, int32_t dim, int64_t out_count,
+                          void* workspace, int64_t workspace_bytes,
+                          asc_stream_t stream);
 
 /* ---- RMS norm -------------------------------------------------------------------
  * asc2.rms_norm(input, gamma, epsilon) (python/asc/language/tile/unary_ops.py:

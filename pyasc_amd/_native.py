@@ -51,7 +51,8 @@ class LaunchPlan(ctypes.Structure):
         return ctypes.string_at(ctypes.addressof(self.args), self.args_size)
 
 
-# name -> argtypes; every entry point returns int32_t.
+# name -> argtypes; every entry point returns int32_t (asc_reduce_f32_workspace a byte
+# count, the others a status).
 SIGNATURES = {
     "asc_device_info": [_c_i32, ctypes.POINTER(_c_i32), ctypes.POINTER(_c_i32), ctypes.POINTER(_c_i32),
                         ctypes.c_char_p],
@@ -67,6 +68,8 @@ SIGNATURES = {
     "asc_gelu_rows_f32": [_c_p, _c_p, _c_i64, _c_i64, _c_i32, _c_i32, _c_i32, _c_p],
     "asc_softmax_rows_f32": [_c_p, _c_p, _c_i64, _c_i64, _c_i32, _c_i32, _c_p],
     "asc_reduce_f32": [_c_i32, _c_p, _c_p, _c_i64, _c_i64, _c_i32, _c_i64, _c_p],
+    "asc_reduce_f32_workspace": [_c_i64, _c_i64, _c_i32],
+    "asc_reduce_f32_ws": [_c_i32, _c_p, _c_p, _c_i64, _c_i64, _c_i32, _c_i64, _c_p, _c_i64, _c_p],
     "asc_rms_norm": [_c_i32, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i32, _c_f32, _c_p],
     "asc_softmax_blocks_f32": [_c_p, _c_p, _c_i64, _c_i64, _c_i32, _c_i32, _c_p],
     "asc_softmax_rows_f16": [_c_p, _c_p, _c_i64, _c_i64, _c_i32, _c_i32, _c_p],

@@ -6,10 +6,14 @@
 // dim 1 (one result per row), dim 0 (one per column) or over all elements
 // (the scalar broadcast into an output by asc2.full).  fp32 accumulation; max
 // and min return the larger / smaller non-NaN operand (IEEE maxNum / minNum).
-//   dim 1: a wave per row, 16-byte loads, in-lane accumulation, DPP/permlane
-//          combine (HBM-bound: 4 B per element).
-//   dim 0: a thread per column walking the rows (coalesced across threads).
+//   dim 1: a wave per row, or a workgroup per row when there are few long rows; 16-byte
+//          loads at element alignment, in-lane accumulation, DPP/permlane combine
+//          (HBM-bound: 4 B per element).
+//   dim 0: a workgroup per 64 columns walks the rows, 64 at a time, 16 bytes per lane.
 //   all:   one 1024-thread block.
+// Few results leave most CUs idle: asc_reduce_f32_ws, with a workspace, splits the rows (dim
+// 0) or the elements (all) over enough workgroups to fill the chip, and a second launch
+// combines their partial results in a fixed order.
 //
 // asc_rms_norm covers asc2.rms_norm (python/asc/language/tile/unary_ops.py:225-237,
 // AscendC RmsNorm): y = x * rsqrt(mean(x^2) + eps) * gamma along the last dim,
@@ -55,81 +59,237 @@ struct ReduceArgs {
   float* out;
   int64_t rows, cols;
   int64_t out_count;  // "all": number of output elements receiving the result
-  bool vec_ok;
 };
 
-// dim 1: rows 4*blockIdx.x + wave; four independent vector loads per lane in
-// flight, then the in-lane partials are combined in a fixed order.
-template <int kOp>
-__global__ void __launch_bounds__(256) reduce_rows_kernel(ReduceArgs p) {
-  const int lane = threadIdx.x & 63;
-  const int64_t r = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (r >= p.rows) return;
-  const float* row = p.x + r * p.cols;
-  const int len = static_cast<int>(p.cols);
+// First element of span i of n elements in `spans` parts, a multiple of 4.
+__device__ __forceinline__ int64_t span_start(int64_t n, int64_t i, int64_t spans) {
+  const int64_t vecs = n / 4;
+  return i == spans ? n : (vecs / spans * i + vecs % spans * i / spans) * 4;
+}
+
+// 16 bytes of fp32 at element alignment, streamed once.
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ f32x4_u load4(const float* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const f32x4_u*>(p));
+}
+
+// Elements [0, len) of x by the kThreads threads of a group (t: the thread's index in it):
+// kUnroll independent vector loads per lane in flight, in-lane partials combined in a fixed order.
+template <int kOp, int kThreads, int kUnroll>
+__device__ __forceinline__ float reduce_span(const float* x, int64_t len, int t) {
   float acc[4] = {identity<kOp>(), identity<kOp>(), identity<kOp>(), identity<kOp>()};
-  const int nvec = len / 4;
-  int q = lane;
-  if (p.vec_ok) {
-    for (; q + 192 < nvec; q += 256) {
-      float4 v[4];
+  const int64_t nvec = len / 4;
+  int64_t q = t;
+  for (; q + (kUnroll - 1) * kThreads < nvec; q += kUnroll * kThreads) {
+    f32x4_u v[kUnroll];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = asc::rows::load_vec(row, q + 64 * u, len, true, identity<kOp>());
+    for (int u = 0; u < kUnroll; ++u) v[u] = load4(x + 4 * (q + u * kThreads));
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        acc[u] = combine<kOp>(acc[u], combine<kOp>(combine<kOp>(v[u].x, v[u].y), combine<kOp>(v[u].z, v[u].w)));
-    }
+    for (int u = 0; u < kUnroll; ++u)
+      acc[u % 4] = combine<kOp>(acc[u % 4], combine<kOp>(combine<kOp>(v[u].x, v[u].y), combine<kOp>(v[u].z, v[u].w)));
   }
-  // remaining vectors (and every element when the row is not 16-byte aligned)
-  for (int e = q * 4; e < len; e += 256) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (e + i < len) acc[i] = combine<kOp>(acc[i], row[e + i]);
+  for (; q < nvec; q += kThreads) {
+    const f32x4_u v = load4(x + 4 * q);
+    acc[0] = combine<kOp>(acc[0], combine<kOp>(combine<kOp>(v.x, v.y), combine<kOp>(v.z, v.w)));
   }
-  const float t = combine<kOp>(combine<kOp>(acc[0], acc[1]), combine<kOp>(acc[2], acc[3]));
-  const float total = wave_combine<kOp>(t);
-  if (lane == 0) p.out[r] = total;
+  if (nvec * 4 + t < len) acc[1] = combine<kOp>(acc[1], x[nvec * 4 + t]);  // at most 3 elements
+  return combine<kOp>(combine<kOp>(acc[0], acc[1]), combine<kOp>(acc[2], acc[3]));
 }
 
-// dim 0: thread per column, rows in order.
-template <int kOp>
-__global__ void __launch_bounds__(256) reduce_cols_kernel(ReduceArgs p) {
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (c >= p.cols) return;
-  float acc = identity<kOp>();
-  for (int64_t r = 0; r < p.rows; ++r) acc = combine<kOp>(acc, p.x[r * p.cols + c]);
-  p.out[c] = acc;
-}
-
-// all elements: one block; the result is written to out[0 .. out_count).
-template <int kOp>
-__global__ void __launch_bounds__(1024) reduce_all_kernel(ReduceArgs p) {
-  __shared__ float part[16];
-  const int64_t n = p.rows * p.cols;
-  float acc = identity<kOp>();
-  for (int64_t i = threadIdx.x; i < n; i += 1024) acc = combine<kOp>(acc, p.x[i]);
-  acc = wave_combine<kOp>(acc);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = acc;
+// Combines one value per thread of a kThreads-thread workgroup; every thread gets the result.
+template <int kOp, int kThreads>
+__device__ __forceinline__ float block_combine(float v) {
+  __shared__ float part[kThreads / 64];
+  v = wave_combine<kOp>(v);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
   __syncthreads();
   float total = part[0];
 #pragma unroll
-  for (int w = 1; w < 16; ++w) total = combine<kOp>(total, part[w]);
+  for (int w = 1; w < kThreads / 64; ++w) total = combine<kOp>(total, part[w]);
+  return total;
+}
+
+// dim 1, a wave per row: rows 4*blockIdx.x + wave.
+template <int kOp>
+__global__ void __launch_bounds__(256) reduce_rows_kernel(ReduceArgs p) {
+  const int64_t r = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (r >= p.rows) return;
+  const float total = wave_combine<kOp>(reduce_span<kOp, 64, 4>(p.x + r * p.cols, p.cols, threadIdx.x & 63));
+  if ((threadIdx.x & 63) == 0) p.out[r] = total;
+}
+
+// dim 1, a workgroup per row.
+template <int kOp>
+__global__ void __launch_bounds__(1024) reduce_long_rows_kernel(ReduceArgs p) {
+  const int64_t r = blockIdx.x;
+  const float total = block_combine<kOp, 1024>(reduce_span<kOp, 1024, 4>(p.x + r * p.cols, p.cols, threadIdx.x));
+  if (threadIdx.x == 0) p.out[r] = total;
+}
+
+// dim 0: workgroup (b, s) reduces rows [s*p.rows/splits, (s+1)*p.rows/splits) of columns 64b ..
+// 64b+63 into out[s * cols + column].  Sixteen lanes cover 256 bytes of a row, a pass of the
+// workgroup 64 rows, four passes' loads in flight.  Bound by HBM once every CU has a
+// workgroup: 16384x4096 47-49 us (5.5-5.7 TB/s) with 256 workgroups of 64 columns, 57 with 32
+// columns (128-byte pieces of rows), 69 with 128 workgroups; 65536x1024 47-51 us.  A thread per
+// column took 6129 and 25088 us: one load in flight on 16 and 4 workgroups.
+constexpr int kColsPerBlock = 64;
+template <int kOp>
+__global__ void __launch_bounds__(1024) reduce_cols_kernel(ReduceArgs p) {
+  __shared__ float4 part[16][16];
+  const int t = threadIdx.x, lane_c = t & 15;
+  const int64_t c = static_cast<int64_t>(blockIdx.x) * kColsPerBlock + lane_c * 4;
+  const int64_t r0 = p.rows * blockIdx.y / gridDim.y, r1 = p.rows * (blockIdx.y + 1) / gridDim.y;
+  const int left = static_cast<int>(p.cols - c < 4 ? p.cols - c : 4);  // columns of this lane
+  float acc[4] = {identity<kOp>(), identity<kOp>(), identity<kOp>(), identity<kOp>()};
+  int64_t r = r0 + (t >> 4);
+  if (left == 4) {
+    const float* x = p.x + c;
+    constexpr int kUnroll = 4;
+    for (; r + (kUnroll - 1) * 64 < r1; r += kUnroll * 64) {
+      f32x4_u v[kUnroll];
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) v[u] = load4(x + (r + u * 64) * p.cols);
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = combine<kOp>(acc[i], v[u][i]);
+    }
+    for (; r < r1; r += 64) {
+      const f32x4_u v = load4(x + r * p.cols);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = combine<kOp>(acc[i], v[i]);
+    }
+  } else if (left > 0) {
+    for (; r < r1; r += 64)
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        if (i < left) acc[i] = combine<kOp>(acc[i], p.x[r * p.cols + c + i]);
+  }
+  // the wave's four rows, then the sixteen waves
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    acc[i] = combine<kOp>(acc[i], asc::lane_xor16(acc[i]));
+    acc[i] = combine<kOp>(acc[i], asc::lane_xor32(acc[i]));
+  }
+  if ((t & 63) < 16) part[t >> 6][lane_c] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  __syncthreads();
+  if (t < kColsPerBlock) {
+    const float* column = reinterpret_cast<const float*>(part) + t;
+    float total = column[0];
+#pragma unroll
+    for (int w = 1; w < 16; ++w) total = combine<kOp>(total, column[w * kColsPerBlock]);
+    const int64_t out_c = static_cast<int64_t>(blockIdx.x) * kColsPerBlock + t;
+    if (out_c < p.cols) p.out[blockIdx.y * p.cols + out_c] = total;
+  }
+}
+
+// dim 0 of few rows or very many columns: four columns per thread, eight rows' loads in flight.
+template <int kOp>
+__global__ void __launch_bounds__(256) reduce_wide_cols_kernel(ReduceArgs p) {
+  const int64_t c = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
+  if (c >= p.cols) return;
+  float acc[4] = {identity<kOp>(), identity<kOp>(), identity<kOp>(), identity<kOp>()};
+  const int left = static_cast<int>(p.cols - c < 4 ? p.cols - c : 4);
+  const float* x = p.x + c;
+  if (left < 4) {
+    for (int64_t r = 0; r < p.rows; ++r)
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        if (i < left) acc[i] = combine<kOp>(acc[i], x[r * p.cols + i]);
+  } else {
+    int64_t r = 0;
+    for (; r + 7 < p.rows; r += 8) {
+      f32x4_u v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = load4(x + (r + u) * p.cols);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = combine<kOp>(acc[i], v[u][i]);
+    }
+    for (; r < p.rows; ++r) {
+      const f32x4_u v = load4(x + r * p.cols);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = combine<kOp>(acc[i], v[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (i < left) p.out[c + i] = acc[i];
+}
+
+// all elements: workgroup s reduces elements [s*n/grid, (s+1)*n/grid); the result is written to
+// out[0 .. out_count), or with several workgroups to out[s].
+template <int kOp>
+__global__ void __launch_bounds__(1024) reduce_all_kernel(ReduceArgs p) {
+  const int64_t n = p.rows * p.cols;
+  const int64_t e0 = span_start(n, blockIdx.x, gridDim.x), e1 = span_start(n, blockIdx.x + 1, gridDim.x);
+  const float total = block_combine<kOp, 1024>(reduce_span<kOp, 1024, 4>(p.x + e0, e1 - e0, threadIdx.x));
+  if (gridDim.x > 1) {
+    if (threadIdx.x == 0) p.out[blockIdx.x] = total;
+    return;
+  }
   for (int64_t i = threadIdx.x; i < p.out_count; i += 1024) p.out[i] = total;
 }
 
+// dim 0 by a thread per four columns: with fewer than 32 rows most of a 64-row pass would be
+// idle, and from 2^18 columns up those threads fill the chip.
+bool wide_cols(int64_t rows, int64_t cols) { return rows < 32 || cols >= (int64_t{1} << 18); }
+
+// Workgroups that a reduction's rows (dim 0) or elements (all) are split over when it has a
+// workspace; 1: no second launch.  A second launch costs about 3 us: it pays from about 1 MiB
+// of input.  256 workgroups, one per CU, are as fast as more of them (16384x4096, column sums
+// and all elements: 47.1 and 44.9 us with 256, 48.7 and 47.9 with 512).
+constexpr int64_t kSplitMinElems = int64_t{1} << 18;
+constexpr int64_t kSplitGroups = 256;
+int64_t reduce_splits(int64_t rows, int64_t cols, int dim) {
+  const int64_t n = rows * cols;
+  if (n < kSplitMinElems || dim == 1) return 1;
+  if (dim == -1) return n / 16384 < kSplitGroups ? n / 16384 : kSplitGroups;
+  if (wide_cols(rows, cols)) return 1;
+  const int64_t col_groups = asc::ceil_div(cols, kColsPerBlock);
+  const int64_t by_groups = kSplitGroups / col_groups, by_rows = rows / 512;
+  const int64_t splits = by_groups < by_rows ? by_groups : by_rows;
+  return splits < 1 ? 1 : splits;
+}
+
 template <int kOp>
-int32_t launch_reduce(const ReduceArgs& p, int dim, hipStream_t s) {
+void launch_cols(const ReduceArgs& p, int64_t splits, hipStream_t s) {
+  const dim3 grid(static_cast<uint32_t>(asc::ceil_div(p.cols, kColsPerBlock)), static_cast<uint32_t>(splits));
+  hipLaunchKernelGGL(reduce_cols_kernel<kOp>, grid, dim3(1024), 0, s, p);
+}
+
+// ws: room for the partial results of `splits` groups (null: splits is 1)
+template <int kOp>
+int32_t launch_reduce(const ReduceArgs& p, int dim, int64_t splits, float* ws, hipStream_t s) {
   if (dim == 1) {
-    // four rows per 256-thread workgroup; one dispatch covers fewer than 2^32 threads
-    const int64_t blocks = asc::ceil_div(p.rows, 4);
+    // A wave per row keeps HBM busy from about 1024 rows up (16384x4096: 6.4 TB/s); fewer rows
+    // of 2048 columns or more take a workgroup each.  One dispatch covers fewer than 2^32 threads.
+    const bool wave_rows = p.rows >= 1024 || p.cols < 2048;
+    const int64_t blocks = wave_rows ? asc::ceil_div(p.rows, 4) : p.rows;
     ASC_REQUIRE(blocks * 256 < (int64_t{1} << 32), ASC_ERR_UNSUPPORTED, "asc_reduce_f32: %lld rows exceed one launch",
                 static_cast<long long>(p.rows));
-    hipLaunchKernelGGL(reduce_rows_kernel<kOp>, dim3(static_cast<uint32_t>(blocks)), dim3(256), 0, s, p);
+    if (wave_rows) {
+      hipLaunchKernelGGL(reduce_rows_kernel<kOp>, dim3(static_cast<uint32_t>(blocks)), dim3(256), 0, s, p);
+    } else {
+      hipLaunchKernelGGL(reduce_long_rows_kernel<kOp>, dim3(static_cast<uint32_t>(blocks)), dim3(1024), 0, s, p);
+    }
   } else if (dim == 0) {
-    hipLaunchKernelGGL(reduce_cols_kernel<kOp>, dim3(static_cast<uint32_t>(asc::ceil_div(p.cols, 256))), dim3(256),
-                       0, s, p);
-  } else {
+    if (wide_cols(p.rows, p.cols)) {
+      hipLaunchKernelGGL(reduce_wide_cols_kernel<kOp>, dim3(static_cast<uint32_t>(asc::ceil_div(p.cols, 1024))),
+                         dim3(256), 0, s, p);
+    } else if (splits == 1) {
+      launch_cols<kOp>(p, 1, s);
+    } else {
+      launch_cols<kOp>(ReduceArgs{p.x, ws, p.rows, p.cols, 0}, splits, s);
+      launch_cols<kOp>(ReduceArgs{ws, p.out, splits, p.cols, 0}, 1, s);
+    }
+  } else if (splits == 1) {
     hipLaunchKernelGGL(reduce_all_kernel<kOp>, dim3(1), dim3(1024), 0, s, p);
+  } else {
+    hipLaunchKernelGGL(reduce_all_kernel<kOp>, dim3(static_cast<uint32_t>(splits)), dim3(1024), 0, s,
+                       ReduceArgs{p.x, ws, p.rows, p.cols, 0});
+    hipLaunchKernelGGL(reduce_all_kernel<kOp>, dim3(1), dim3(1024), 0, s, ReduceArgs{ws, p.out, 1, splits, p.out_count});
   }
   return asc::check_launch("asc_reduce_f32");
 }
@@ -322,8 +482,9 @@ int32_t launch_rms(const RmsArgs& p, hipStream_t s) {
 
 }  // namespace
 
-extern "C" int32_t asc_reduce_f32(int32_t op, const float* x, float* out, int64_t rows, int64_t cols, int32_t dim,
-                                  int64_t out_count, asc_stream_t stream) {
+extern "C" int32_t asc_reduce_f32_ws(int32_t op, const float* x, float* out, int64_t rows, int64_t cols, int32_t dim,
+                                     int64_t out_count, void* workspace, int64_t workspace_bytes,
+                                     asc_stream_t stream) {
   ASC_REQUIRE(op >= kSum && op <= kProd, ASC_ERR_INVALID_ARG, "asc_reduce_f32: op must be 0..3, got %d", op);
   ASC_REQUIRE(dim == 0 || dim == 1 || dim == -1, ASC_ERR_INVALID_ARG,
               "asc_reduce_f32: dim must be 0, 1 or -1 (all), got %d", dim);
@@ -333,14 +494,37 @@ extern "C" int32_t asc_reduce_f32(int32_t op, const float* x, float* out, int64_
   if (results == 0) return ASC_OK;
   ASC_REQUIRE(rows > 0 && cols > 0, ASC_ERR_INVALID_ARG, "asc_reduce_f32: empty input");
   ASC_REQUIRE(x && out, ASC_ERR_INVALID_ARG, "asc_reduce_f32: null buffer");
-  ReduceArgs p{x, out, rows, cols, out_count, asc::aligned16(x) && (cols % 4) == 0};
+  const ReduceArgs p{x, out, rows, cols, out_count};
+  int64_t splits = 1;
+  if (workspace != nullptr) {
+    splits = reduce_splits(rows, cols, dim);
+    const int64_t need = asc_reduce_f32_workspace(rows, cols, dim);
+    ASC_REQUIRE(workspace_bytes >= need, ASC_ERR_INVALID_ARG,
+                "asc_reduce_f32_ws: the partial results need %lld bytes, the workspace holds %lld", (long long)need,
+                (long long)workspace_bytes);
+    ASC_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 3) == 0, ASC_ERR_ALIGNMENT,
+                "asc_reduce_f32_ws: the workspace must be 4-byte aligned");
+  }
+  float* ws = static_cast<float*>(workspace);
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (op) {
-    case kSum: return launch_reduce<kSum>(p, dim, s);
-    case kMax: return launch_reduce<kMax>(p, dim, s);
-    case kMin: return launch_reduce<kMin>(p, dim, s);
-    default: return launch_reduce<kProd>(p, dim, s);
+    case kSum: return launch_reduce<kSum>(p, dim, splits, ws, s);
+    case kMax: return launch_reduce<kMax>(p, dim, splits, ws, s);
+    case kMin: return launch_reduce<kMin>(p, dim, splits, ws, s);
+    default: return launch_reduce<kProd>(p, dim, splits, ws, s);
   }
+}
+
+extern "C" int32_t asc_reduce_f32_workspace(int64_t rows, int64_t cols, int32_t dim) {
+  if (rows <= 0 || cols <= 0) return 0;
+  const int64_t splits = reduce_splits(rows, cols, dim);
+  // dim 0: splits * ceil(cols / 64) <= 256, so this never exceeds 64 KiB
+  return splits == 1 ? 0 : static_cast<int32_t>(splits * (dim == 0 ? cols : 1) * static_cast<int64_t>(sizeof(float)));
+}
+
+extern "C" int32_t asc_reduce_f32(int32_t op, const float* x, float* out, int64_t rows, int64_t cols, int32_t dim,
+                                  int64_t out_count, asc_stream_t stream) {
+  return asc_reduce_f32_ws(op, x, out, rows, cols, dim, out_count, nullptr, 0, stream);
 }
 
 extern "C" int32_t asc_rms_norm(int32_t dtype, const void* x, const float* gamma, void* out, int64_t num_rows,

@@ -40,6 +40,13 @@ def _device_tensor(t: Any, name: str) -> torch.Tensor:
     return t
 
 
+def _keep_for_stream(workspace: torch.Tensor, handle: int) -> None:
+    """A workspace is freed when its call returns: on a stream other than torch's current one
+    the caching allocator must not hand its memory out again before the launches have run."""
+    if handle != torch.cuda.current_stream(workspace.device).cuda_stream:
+        workspace.record_stream(torch.cuda.ExternalStream(handle, device=workspace.device))
+
+
 def _contiguous(t: torch.Tensor, name: str) -> torch.Tensor:
     if not t.is_contiguous():
         raise ValueError(f"'{name}' must be contiguous")
@@ -256,16 +263,34 @@ def reduce_f32(x: torch.Tensor, out: torch.Tensor, op: str, dim: Optional[int], 
     else:
         raise ValueError("x must be 1-D or 2-D")
     if dim is None:
-        _native.call("asc_reduce_f32", REDUCE_OPS[op], x.data_ptr(), out.data_ptr(), rows, cols, -1, out.numel(),
-                     _stream(stream))
+        _reduce(x, out, op, rows, cols, -1, out.numel(), stream)
         return
     if x.dim() != 2 or dim not in (0, 1):
         raise ValueError(f"dim must be 0 or 1 of a 2-D tensor, got dim={dim} for shape {tuple(x.shape)}")
     need = rows if dim == 1 else cols
     if out.numel() != need:
         raise ValueError(f"out must hold {need} elements, holds {out.numel()}")
-    _native.call("asc_reduce_f32", REDUCE_OPS[op], x.data_ptr(), out.data_ptr(), rows, cols, dim, need,
-                 _stream(stream))
+    _reduce(x, out, op, rows, cols, dim, need, stream)
+
+
+# below this many elements no reduction uses a workspace (kSplitMinElems of csrc/reduce.hip)
+_REDUCE_SPLIT_MIN = 1 << 18
+
+
+def _reduce(x: torch.Tensor, out: torch.Tensor, op: str, rows: int, cols: int, dim: int, count: int, stream) -> None:
+    """One reduction; one with few results over many elements gets a workspace (at most 64 KiB)
+    from torch's allocator on the launch stream for its partial results."""
+    handle = _stream(stream)
+    args = (REDUCE_OPS[op], x.data_ptr(), out.data_ptr(), rows, cols, dim, count)
+    nbytes = 0
+    if dim != 1 and rows * cols >= _REDUCE_SPLIT_MIN:
+        nbytes = _native.load_library().asc_reduce_f32_workspace(rows, cols, dim)
+    if nbytes == 0:
+        _native.call("asc_reduce_f32", *args, handle)
+        return
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    _keep_for_stream(workspace, handle)
+    _native.call("asc_reduce_f32_ws", *args, workspace.data_ptr(), nbytes, handle)
 
 
 def rms_norm(x: torch.Tensor, gamma: torch.Tensor, out: torch.Tensor, num_rows: int, num_cols: int,
@@ -377,10 +402,7 @@ def matmul_chained(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, workspace:
     handle = _stream(stream)
     if workspace is None:
         workspace = torch.empty(M * N, dtype=a.dtype, device=a.device)
-        # freed on return: on a stream other than torch's current one the caching
-        # allocator must not hand its memory out again before these launches have run
-        if handle != torch.cuda.current_stream(a.device).cuda_stream:
-            workspace.record_stream(torch.cuda.ExternalStream(handle, device=a.device))
+        _keep_for_stream(workspace, handle)
     else:
         _contiguous(_device_tensor(workspace, "workspace"), "workspace")
     nbytes = workspace.numel() * workspace.element_size()
