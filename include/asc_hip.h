@@ -212,9 +212,9 @@ int32_t asc_softmax_blocks_f16(const void* x, void* out, int64_t num_rows,
                                int64_t num_cols, int32_t block_size,
                                int32_t grid, asc_stream_t stream);
 
-/* The launch the four softmax entries above make, for a launcher that runs the
- * same kernels from the code object pyasc_amd/lib/co/asc2_softmax.hsaco instead
- * (the asc2 launch path does, through asc_module_launch).  No counterpart in the
+/* A launch of the four softmax entries above, chosen by dtype and row length, for
+ * a launcher that runs the kernels from the code object
+ * pyasc_amd/lib/co/asc2_softmax.hsaco through asc_module_launch.  No counterpart in the
  * reference, whose compiler fixes the launch inside the kernel binary.
  * dtype ASC_DT_FLOAT32 / FLOAT16; fused 0 for asc_softmax_rows_* (size is
  * tile_size), 1 for asc_softmax_blocks_* (size is block_size); the other
@@ -235,6 +235,13 @@ typedef struct asc_softmax_plan {
 int32_t asc_softmax_plan(int32_t dtype, int32_t fused, const void* x,
                          const void* out, int64_t num_rows, int64_t num_cols,
                          int32_t size, int32_t grid, asc_softmax_plan_t* plan);
+/* The launch the four entries make: asc_softmax_plan's, or for few or long rows
+ * the same softmax with 1024 threads per row, and for short float16 rows a grid
+ * of no more workgroups than the rows need.  Same arguments and errors. */
+int32_t asc_softmax_dispatch(int32_t dtype, int32_t fused, const void* x,
+                             const void* out, int64_t num_rows,
+                             int64_t num_cols, int32_t size, int32_t grid,
+                             asc_softmax_plan_t* plan);
 
 /* ---- reductions ---------------------------------------------------------------
  * asc2.reduce_sum / reduce_max / reduce_min / reduce_prod

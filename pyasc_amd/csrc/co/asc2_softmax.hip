@@ -6,8 +6,8 @@
 // softmax_kernels.h, with C names (asc2_softmax_<body>) for hipModuleGetFunction;
 // every kernel takes
 //   (const void* x, void* out, int64_t rows, int64_t stride, int32_t len, int32_t flag)
-// and asc_softmax_plan names the kernel, grid, block and arguments of a launch,
-// the same plan the library's asc_softmax_* entries launch.
+// and asc_softmax_dispatch names the kernel, grid, block and arguments of the
+// launch the library's asc_softmax_* entries make.
 #include "softmax_kernels.h"
 
 ASC_SOFTMAX_KERNELS(extern "C", asc2_softmax_)

@@ -1,5 +1,5 @@
-// Row access for the row kernels (softmax.hip, reduce.hip): a row of fp32
-// values held in registers as float4 vectors.
+// Row access for the softmax kernels: a row of fp32 values held in registers as float4
+// vectors.
 #pragma once
 
 #include "common.h"
@@ -7,7 +7,9 @@
 namespace asc {
 namespace rows {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+// 16 bytes at element alignment: a row of any length starts on an element, and gfx950 loads
+// and stores 16 bytes there in one instruction (a wave's row piece touches one line more).
+typedef float f32x4 __attribute__((ext_vector_type(4), aligned(4)));
 
 struct RowView {
   const float* x;
@@ -15,13 +17,12 @@ struct RowView {
   int64_t rows;    // covered rows [0, rows)
   int64_t stride;  // elements between row starts
   int32_t len;     // columns processed per row
-  bool vec_ok;     // rows start 16-byte aligned
 };
 
 // Vector q (elements 4q..4q+3) of a row, `pad` past `len`.
-__device__ __forceinline__ float4 load_vec(const float* row, int q, int len, bool vec_ok, float pad) {
+__device__ __forceinline__ float4 load_vec(const float* row, int q, int len, float pad) {
   const int e = q * 4;
-  if (vec_ok && e + 3 < len) {
+  if (e + 3 < len) {
     // streamed once: non-temporal so the rows do not displace other cached data
     const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(row + e));
     return make_float4(v.x, v.y, v.z, v.w);
@@ -34,9 +35,9 @@ __device__ __forceinline__ float4 load_vec(const float* row, int q, int len, boo
   return v;
 }
 
-__device__ __forceinline__ void store_vec(float* row, int q, int len, bool vec_ok, float4 v) {
+__device__ __forceinline__ void store_vec(float* row, int q, int len, float4 v) {
   const int e = q * 4;
-  if (vec_ok && e + 3 < len) {
+  if (e + 3 < len) {
     __builtin_nontemporal_store(f32x4{v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4*>(row + e));
     return;
   }
@@ -53,28 +54,28 @@ __device__ __forceinline__ void store_vec(float* row, int q, int len, bool vec_o
 // tail takes the per-lane path.  (A per-lane choice between the two load
 // forms would run both and serialise the loads on their shared registers.)
 template <int N, int kStride>
-__device__ __forceinline__ void load_row(float4 (&v)[N], const float* row, int q0, int len, bool vec_ok, float pad) {
+__device__ __forceinline__ void load_row(float4 (&v)[N], const float* row, int q0, int len, float pad) {
 #pragma unroll
   for (int j = 0; j < N; ++j) {
     const int q = q0 + kStride * j;
-    if (vec_ok && kStride * (j + 1) * 4 <= len) {
-      const f32x4 t = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(row) + q);
+    if (kStride * (j + 1) * 4 <= len) {
+      const f32x4 t = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(row + 4 * q));
       v[j] = make_float4(t.x, t.y, t.z, t.w);
     } else {
-      v[j] = load_vec(row, q, len, vec_ok, pad);
+      v[j] = load_vec(row, q, len, pad);
     }
   }
 }
 
 template <int N, int kStride>
-__device__ __forceinline__ void store_row(const float4 (&v)[N], float* row, int q0, int len, bool vec_ok) {
+__device__ __forceinline__ void store_row(const float4 (&v)[N], float* row, int q0, int len) {
 #pragma unroll
   for (int j = 0; j < N; ++j) {
     const int q = q0 + kStride * j;
-    if (vec_ok && kStride * (j + 1) * 4 <= len) {
-      __builtin_nontemporal_store(f32x4{v[j].x, v[j].y, v[j].z, v[j].w}, reinterpret_cast<f32x4*>(row) + q);
+    if (kStride * (j + 1) * 4 <= len) {
+      __builtin_nontemporal_store(f32x4{v[j].x, v[j].y, v[j].z, v[j].w}, reinterpret_cast<f32x4*>(row + 4 * q));
     } else {
-      store_vec(row, q, len, vec_ok, v[j]);
+      store_vec(row, q, len, v[j]);
     }
   }
 }

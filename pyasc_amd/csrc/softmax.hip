@@ -1,8 +1,8 @@
 // Row softmax for the two asc2 softmax kernels (python/test/asc2/kernels/):
 //   test_softmax.py:16-27        grid-stride rows, one [1, tile_size] tile per row
 //   test_softmax_fused.py:16-24  contiguous row blocks through asc2.softmax
-// The device bodies are in softmax_kernels.h.  This file holds the launch plan
-// (asc_softmax_plan: which body, its grid and block, its six arguments), which
+// The device bodies are in softmax_kernels.h.  This file holds the launch choice
+// (asc_softmax_dispatch: which body, its grid and block, its six arguments), which
 // the library's entry points and the asc2 code-object launch path share, and
 // the library's own instances of the kernels.
 #include "softmax_kernels.h"
@@ -22,6 +22,9 @@ enum Kernel : int32_t {
   kF16,
   kPaddedF32,
   kPaddedF16,
+  kShortF32,
+  kWideF32,
+  kWideF16,
   kNumKernels
 };
 
@@ -32,11 +35,13 @@ using KernelFn = void (*)(const void*, void*, int64_t, int64_t, int32_t, int32_t
 const KernelFn kKernels[kNumKernels] = {softmax_wave_1x2,    softmax_wave_2x2,    softmax_block_2x128,
                                         softmax_block_2x256, softmax_block_2x512, softmax_block_8x256,
                                         softmax_long,        softmax_f16,         softmax_padded_f32,
-                                        softmax_padded_f16};
+                                        softmax_padded_f16,  softmax_short_f32,   softmax_wide_f32,
+                                        softmax_wide_f16};
 const char* const kCodeObjectNames[kNumKernels] = {
     "asc2_softmax_wave_1x2",    "asc2_softmax_wave_2x2",    "asc2_softmax_block_2x128", "asc2_softmax_block_2x256",
     "asc2_softmax_block_2x512", "asc2_softmax_block_8x256", "asc2_softmax_long",        "asc2_softmax_f16",
-    "asc2_softmax_padded_f32",  "asc2_softmax_padded_f16"};
+    "asc2_softmax_padded_f32",  "asc2_softmax_padded_f16",  "asc2_softmax_short_f32",   "asc2_softmax_wide_f32",
+    "asc2_softmax_wide_f16"};
 
 struct Plan {
   Kernel kernel = kNumKernels;
@@ -140,6 +145,30 @@ int32_t make_plan(bool half, bool fused, const void* x, const void* out, int64_t
   return ASC_OK;
 }
 
+// The launch the entries make of make_plan's.  fp32 rows of up to 512 columns take 16 lanes each
+// once there are enough to fill the chip that way (2100x256: 3.6 us with a wave per two rows, 3.1
+// with 16 lanes; 500 rows make 32 such workgroups, and either takes 3 us).  Rows
+// that 256 threads cannot hold take 1024 (figures at wide_body; fp16 2000x32000: 101 us with
+// 256, 63 with 1024), and no more workgroups are launched for fp16 than its rows fill
+// (100000x64: 25 us with the plan's 65536, most of them empty, 12.4 with 6250).
+void dispatch(Plan& p) {
+  if (p.grid == 0) return;
+  const bool fits = p.rows * 1024 <= static_cast<int64_t>(UINT32_MAX);
+  if ((p.kernel == kWave1x2 || p.kernel == kWave2x2) && p.len <= 512 && p.rows > 1024) {
+    p.kernel = kShortF32;
+    p.grid = asc::ceil_div(p.rows, 16);
+  } else if (p.kernel == kLong && fits && p.len > 16384) {
+    p.kernel = kWideF32;
+    p.block = 1024;
+  } else if (p.kernel == kF16 && fits && p.len > 16377) {
+    p.kernel = kWideF16;
+    p.block = 1024;
+  } else if (p.kernel == kF16) {
+    const int64_t groups = asc::ceil_div(p.rows, asc::softmax::f16_rows_per_block(p.len, p.rows));
+    if (groups < p.grid) p.grid = groups;
+  }
+}
+
 int32_t launch(const Plan& p, asc_stream_t stream, const char* who) {
   if (p.grid == 0) return ASC_OK;
   hipLaunchKernelGGL(kKernels[p.kernel], dim3(static_cast<uint32_t>(p.grid)), dim3(p.block), 0,
@@ -151,7 +180,9 @@ int32_t plan_and_launch(bool half, bool fused, const void* x, void* out, int64_t
                         int32_t size, int32_t grid, asc_stream_t stream, const char* who) {
   Plan p;
   const int32_t rc = make_plan(half, fused, x, out, num_rows, num_cols, size, grid, who, p);
-  return rc != ASC_OK ? rc : launch(p, stream, who);
+  if (rc != ASC_OK) return rc;
+  dispatch(p);
+  return launch(p, stream, who);
 }
 
 }  // namespace
@@ -178,8 +209,10 @@ extern "C" int32_t asc_softmax_blocks_f16(const void* x, void* out, int64_t num_
                          "asc_softmax_blocks_f16");
 }
 
-extern "C" int32_t asc_softmax_plan(int32_t dtype, int32_t fused, const void* x, const void* out, int64_t num_rows,
-                                    int64_t num_cols, int32_t size, int32_t grid, asc_softmax_plan_t* plan) {
+namespace {
+
+int32_t fill_plan(bool dispatched, int32_t dtype, int32_t fused, const void* x, const void* out, int64_t num_rows,
+                  int64_t num_cols, int32_t size, int32_t grid, asc_softmax_plan_t* plan) {
   ASC_REQUIRE(plan, ASC_ERR_INVALID_ARG, "asc_softmax_plan: null plan");
   ASC_REQUIRE(dtype == ASC_DT_FLOAT32 || dtype == ASC_DT_FLOAT16, ASC_ERR_UNSUPPORTED,
               "asc_softmax_plan: unsupported dtype code %d", dtype);
@@ -189,6 +222,7 @@ extern "C" int32_t asc_softmax_plan(int32_t dtype, int32_t fused, const void* x,
   Plan p;
   const int32_t rc = make_plan(half, fused != 0, x, out, num_rows, num_cols, size, grid, who, p);
   if (rc != ASC_OK) return rc;
+  if (dispatched) dispatch(p);
   *plan = asc_softmax_plan_t{};
   if (p.grid == 0) return ASC_OK;
   __builtin_strncpy(plan->kernel, kCodeObjectNames[p.kernel], sizeof(plan->kernel) - 1);
@@ -199,4 +233,17 @@ extern "C" int32_t asc_softmax_plan(int32_t dtype, int32_t fused, const void* x,
   plan->len = p.len;
   plan->flag = p.flag;
   return ASC_OK;
+}
+
+}  // namespace
+
+extern "C" int32_t asc_softmax_plan(int32_t dtype, int32_t fused, const void* x, const void* out, int64_t num_rows,
+                                    int64_t num_cols, int32_t size, int32_t grid, asc_softmax_plan_t* plan) {
+  return fill_plan(false, dtype, fused, x, out, num_rows, num_cols, size, grid, plan);
+}
+
+extern "C" int32_t asc_softmax_dispatch(int32_t dtype, int32_t fused, const void* x, const void* out,
+                                        int64_t num_rows, int64_t num_cols, int32_t size, int32_t grid,
+                                        asc_softmax_plan_t* plan) {
+  return fill_plan(true, dtype, fused, x, out, num_rows, num_cols, size, grid, plan);
 }

@@ -230,14 +230,24 @@ def softmax_blocks(x: torch.Tensor, out: torch.Tensor, num_rows: int, num_cols: 
 
 def softmax_plan(x: torch.Tensor, out: torch.Tensor, num_rows: int, num_cols: int, size: int, grid: int,
                  fused: bool) -> "_native.SoftmaxPlan":
-    """The launch softmax_rows (fused False, size = tile_size) or softmax_blocks (fused True,
-    size = block_size) makes for these buffers, as a kernel of the asc2_softmax code object
-    with its grid, block and arguments (asc_softmax_plan); plan.grid == 0 when there is
+    """A launch of softmax_rows (fused False, size = tile_size) or softmax_blocks (fused True,
+    size = block_size) chosen by dtype and row length, as a kernel of the asc2_softmax code
+    object with its grid, block and arguments (asc_softmax_plan); plan.grid == 0 when there is
     nothing to launch.  Same checks and errors as those two calls."""
+    return _softmax_plan("asc_softmax_plan", x, out, num_rows, num_cols, size, grid, fused)
+
+
+def softmax_dispatch(x: torch.Tensor, out: torch.Tensor, num_rows: int, num_cols: int, size: int, grid: int,
+                     fused: bool) -> "_native.SoftmaxPlan":
+    """The launch those two calls make (asc_softmax_dispatch), in softmax_plan's form."""
+    return _softmax_plan("asc_softmax_dispatch", x, out, num_rows, num_cols, size, grid, fused)
+
+
+def _softmax_plan(entry: str, x, out, num_rows, num_cols, size, grid, fused) -> "_native.SoftmaxPlan":
     suffix = _softmax_launch(x, out, num_rows, num_cols, size, grid, fused)
     plan = _native.SoftmaxPlan()
-    _native.call("asc_softmax_plan", _native.DT_FLOAT32 if suffix == "f32" else _native.DT_FLOAT16, int(fused),
-                 x.data_ptr(), out.data_ptr(), num_rows, num_cols, size, grid, ctypes.byref(plan))
+    _native.call(entry, _native.DT_FLOAT32 if suffix == "f32" else _native.DT_FLOAT16, int(fused), x.data_ptr(),
+                 out.data_ptr(), num_rows, num_cols, size, grid, ctypes.byref(plan))
     return plan
 
 

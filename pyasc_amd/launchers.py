@@ -188,14 +188,17 @@ def _gelu(call: KernelCall) -> None:
 
 # ------------------------------------------------------------------------------------------- softmax
 
-# The kernels of the asc2_softmax code object (csrc/co/asc2_softmax.hip), one per row body.
+# The kernels of the asc2_softmax code object (csrc/co/asc2_softmax.hip), one per row body:
+# those asc_softmax_plan names, and those only asc_softmax_dispatch does.
 SOFTMAX_CO_FUNCTIONS = tuple(f"asc2_softmax_{body}" for body in (
     "wave_1x2", "wave_2x2", "block_2x128", "block_2x256", "block_2x512", "block_8x256", "long", "f16", "padded_f32",
     "padded_f16"))
+SOFTMAX_DISPATCH_FUNCTIONS = SOFTMAX_CO_FUNCTIONS + tuple(
+    f"asc2_softmax_{name}" for name in ("short_f32", "wide_f32", "wide_f16"))
 
 
 def _softmax_code_object_launch(fused: bool):
-    """softmax_kernel through the asc2_softmax code object: asc_softmax_plan picks the
+    """softmax_kernel through the asc2_softmax code object: asc_softmax_dispatch picks the
     kernel, grid, block and arguments the library entry (asc_softmax_rows_* /
     asc_softmax_blocks_*) would launch, and the code object's kernel of that name runs
     them (the same device body)."""
@@ -203,8 +206,8 @@ def _softmax_code_object_launch(fused: bool):
 
     def launch(call: KernelCall, functions) -> None:
         x, out = call.args["x_ptr"], call.args["out_ptr"]
-        plan = kernels.softmax_plan(x, out, int(call.get("num_rows")), int(call.get("num_cols")),
-                                    int(call.get(size_name)), call.grid, fused)
+        plan = kernels.softmax_dispatch(x, out, int(call.get("num_rows")), int(call.get("num_cols")),
+                                        int(call.get(size_name)), call.grid, fused)
         if plan.grid:
             module.launch(functions[plan.kernel.decode()], plan.grid, plan.block,
                           [("ptr", x.data_ptr()), ("ptr", out.data_ptr()), ("i64", plan.rows),
@@ -213,9 +216,11 @@ def _softmax_code_object_launch(fused: bool):
     return launch
 
 
-SOFTMAX_ROWS_CODE_OBJECT = module.CodeObject("asc2_softmax", SOFTMAX_CO_FUNCTIONS, _softmax_code_object_launch(False),
+SOFTMAX_ROWS_CODE_OBJECT = module.CodeObject("asc2_softmax", SOFTMAX_DISPATCH_FUNCTIONS,
+                                             _softmax_code_object_launch(False),
                                              "pyasc_amd/csrc/co/asc2_softmax.hip")
-SOFTMAX_BLOCKS_CODE_OBJECT = module.CodeObject("asc2_softmax", SOFTMAX_CO_FUNCTIONS, _softmax_code_object_launch(True),
+SOFTMAX_BLOCKS_CODE_OBJECT = module.CodeObject("asc2_softmax", SOFTMAX_DISPATCH_FUNCTIONS,
+                                               _softmax_code_object_launch(True),
                                                "pyasc_amd/csrc/co/asc2_softmax.hip")
 
 
