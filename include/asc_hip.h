@@ -97,7 +97,7 @@ int32_t asc_module_launch(void* function, uint32_t grid, uint32_t block,
 
 /* A launch of one kernel of a prebuilt code object whose argument is a single
  * struct: the kernel's symbol, its grid and block, and the struct's bytes as the
- * argument blob asc_module_launch takes.  asc_flash_attention_plan,
+ * argument blob asc_module_launch takes.  asc_flash_attention_dispatch,
  * asc_matmul_dispatch and asc_matmul_i8_dispatch fill it with exactly the launch
  * their library entry points make.  No counterpart in the reference, whose compiler
  * fixes the launch inside the kernel binary. */
@@ -425,6 +425,14 @@ int32_t asc_flash_attention_plan(const void* q, const void* k, const void* v,
                                  int64_t heads, int64_t seq_len,
                                  int32_t head_dim, float sm_scale,
                                  int32_t causal, asc_launch_plan_t* plan);
+/* The launch asc_flash_attention_fwd_bf16 makes: asc_flash_attention_plan's, or for
+ * few or short heads a kernel that splits the keys over waves.  Same arguments and
+ * errors. */
+int32_t asc_flash_attention_dispatch(const void* q, const void* k, const void* v,
+                                     void* o, float* lse, int64_t batch,
+                                     int64_t heads, int64_t seq_len,
+                                     int32_t head_dim, float sm_scale,
+                                     int32_t causal, asc_launch_plan_t* plan);
 
 /* ---- element-wise tile operations ------------------------------------------------
  * The generic kernels of the reference's operation tests, one op per launch:

@@ -88,6 +88,8 @@ SIGNATURES = {
                                      _c_p],
     "asc_flash_attention_plan": [_c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i32, _c_f32, _c_i32,
                                  ctypes.POINTER(LaunchPlan)],
+    "asc_flash_attention_dispatch": [_c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i32, _c_f32, _c_i32,
+                                     ctypes.POINTER(LaunchPlan)],
     "asc_matmul_plan": [_c_i32, _c_i32, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i32,
                         _c_f32, ctypes.POINTER(LaunchPlan)],
     "asc_matmul_dispatch": [_c_i32, _c_i32, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,

@@ -159,7 +159,8 @@ struct FaState {
   int qw0;  // first query of this wave: q0 + wave * kQ
   float scale_log2;
   __amdgpu_buffer_rsrc_t rsrc_k, rsrc_v;
-  int voff_k[4], voff_v;  // voff_k[i]: this wave's i-th K load (kLoadsPerWave <= 4)
+  static constexpr int kKOffs = kLoadsPerWave < 4 ? kLoadsPerWave : 4;
+  int voff_k[4], voff_v;  // voff_k[i % 4]: this wave's i-th K load
   // Per-lane LDS read offsets, loop-invariant: the K swizzle of row kb*32+col
   // equals that of row col, and the V swizzle of row r0+j (r0 % 4 == 0) equals
   // that of row j, so every other term of a read address is an immediate.
@@ -183,9 +184,9 @@ struct FaState {
     rsrc_v = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(Vh), static_cast<short>(0), bytes, 0x00020000);
     constexpr int kLanesPerRow = 64 / kRowsPerLoad;
     const int rr = lane / kLanesPerRow, pos = lane % kLanesPerRow;
-    static_assert(kLoadsPerWave >= 1 && kLoadsPerWave <= 4, "K load offsets");
+    static_assert(kLoadsPerWave >= 1, "K load offsets");
 #pragma unroll
-    for (int i = 0; i < kLoadsPerWave; ++i) {
+    for (int i = 0; i < kKOffs; ++i) {
       // the K swizzle depends on (row mod 16) = kRowsPerLoad*(R mod 4) + rr; indexing
       // by the load number keeps the array in registers whatever the wave count
       const int R = wave * kLoadsPerWave + i;
@@ -220,7 +221,7 @@ struct FaState {
       const int roff = (k0 + kRowsPerLoad * R) * (D * 2);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(kIsV ? rsrc_v : rsrc_k,
                                                (__attribute__((address_space(3))) void*)(dst + wave_lds + i * 1024),
-                                               16, (kIsV ? voff_v : voff_k[i]) + roff, 0, 0, 0);
+                                               16, (kIsV ? voff_v : voff_k[i & 3]) + roff, 0, 0, 0);
     }
   }
 
@@ -488,11 +489,47 @@ struct FaConfig;
 template <>
 struct FaConfig<128> {
   static constexpr int kWaves = 8, QB = 1, kWgPerCu = 1;
+  static constexpr int kQueries = 32 * QB * kWaves;  // per workgroup
 };
 template <>
 struct FaConfig<64> {
   static constexpr int kWaves = 4, QB = 1, kWgPerCu = 2;
+  static constexpr int kQueries = 32 * QB * kWaves;
 };
+
+// Block order.  Workgroup b runs on XCD b % 8, and each XCD starts its
+// workgroups in order of b / 8.  When the (batch, head) count divides by 8,
+// XCD x takes heads x, x+8, x+16, ... in groups of head_group heads and runs
+// the query blocks of one group back to back, interleaving the group's heads
+// block by block.  The workgroups resident on an XCD at once then stream the
+// same few heads' K/V through that XCD's L2 (fetched from HBM about once per
+// head, instead of once per round of resident query blocks).  Non-causal
+// blocks are all alike and use groups of one head.  Causal blocks run heavy
+// (late) query blocks first, and the host sizes the group so that one group's
+// blocks fill the workgroup slots of the XCD twice over: the heaviest blocks of
+// a group then start together and the lightest end the XCD's run, instead of
+// the last head's heavy blocks starting behind the previous head's light ones.
+// Otherwise: query-block major (heavy first over all heads when causal).
+__device__ __forceinline__ void fa_block(const FaArgs& p, int64_t& bh, int& qblk) {
+  // everything here is at most the grid, which fits 31 bits
+  const uint32_t bid = blockIdx.x;
+  const uint32_t heads = static_cast<uint32_t>(p.heads_total), group = static_cast<uint32_t>(p.head_group);
+  if (heads % 8 == 0) {
+    const uint32_t slot = bid >> 3;  // < heads / 8 * n_qblocks
+    const uint32_t per_group = group * static_cast<uint32_t>(p.n_qblocks);
+    const uint32_t grp = slot / per_group;
+    const uint32_t r = slot - grp * per_group;
+    const uint32_t g0 = grp * group;
+    const uint32_t heads_left = (heads >> 3) - g0;  // >= 1; the last group may be partial
+    const uint32_t gsz = heads_left < group ? heads_left : group;
+    bh = (bid & 7) + 8 * (g0 + r % gsz);
+    qblk = static_cast<int>(r / gsz);
+  } else {
+    bh = bid % heads;
+    qblk = static_cast<int>(bid / heads);
+  }
+  if (p.causal) qblk = p.n_qblocks - 1 - qblk;
+}
 
 // The attention of one workgroup: query block and (batch, head) from the block index.
 template <int D>
@@ -505,7 +542,7 @@ __device__ __forceinline__ void fa_fwd_body(const FaArgs& p) {
   constexpr int kKSteps = St::kKSteps;
   constexpr int kDBlocks = St::kDBlocks;
   constexpr int kThreads = kWaves * 64;
-  constexpr int BQ = St::kQ * kWaves;  // queries per workgroup
+  constexpr int BQ = FaConfig<D>::kQueries;
   // K ring (stages 0-2) and V ring (stages 3-5).  LDS reads of the rings are
   // inline asm with explicit waits, so no compiler alias analysis between DMA
   // and reads is involved.
@@ -521,37 +558,9 @@ __device__ __forceinline__ void fa_fwd_body(const FaArgs& p) {
   st.h = lane >> 5;    // lane half
   const int wave = st.wave, col = st.col, h = st.h;
 
-  // Block order.  Workgroup b runs on XCD b % 8, and each XCD starts its
-  // workgroups in order of b / 8.  When the (batch, head) count divides by 8,
-  // XCD x takes heads x, x+8, x+16, ... in groups of head_group heads and runs
-  // the query blocks of one group back to back, interleaving the group's heads
-  // block by block.  The workgroups resident on an XCD at once then stream the
-  // same few heads' K/V through that XCD's L2 (fetched from HBM about once per
-  // head, instead of once per round of resident query blocks).  Non-causal
-  // blocks are all alike and use groups of one head.  Causal blocks run heavy
-  // (late) query blocks first, and the host sizes the group so that one group's
-  // blocks fill the workgroup slots of the XCD twice over: the heaviest blocks of
-  // a group then start together and the lightest end the XCD's run, instead of
-  // the last head's heavy blocks starting behind the previous head's light ones.
-  // Otherwise: query-block major (heavy first over all heads when causal).
-  const int64_t bid = blockIdx.x;
   int64_t bh;
   int qblk;
-  if (p.heads_total % 8 == 0) {
-    const int64_t slot = bid >> 3;  // < heads_total / 8 * n_qblocks
-    const int64_t per_group = static_cast<int64_t>(p.head_group) * p.n_qblocks;
-    const int64_t grp = slot / per_group;
-    const int64_t r = slot - grp * per_group;
-    const int64_t g0 = grp * p.head_group;
-    const int64_t heads_left = (p.heads_total >> 3) - g0;  // >= 1; the last group may be partial
-    const int64_t gsz = heads_left < p.head_group ? heads_left : p.head_group;
-    bh = (bid & 7) + 8 * (g0 + r % gsz);
-    qblk = static_cast<int>(r / gsz);
-  } else {
-    bh = bid % p.heads_total;
-    qblk = static_cast<int>(bid / p.heads_total);
-  }
-  if (p.causal) qblk = p.n_qblocks - 1 - qblk;
+  fa_block(p, bh, qblk);
   const int q0 = qblk * BQ;
   const int S = p.seq;
   const int64_t head_off = bh * static_cast<int64_t>(S) * D;
@@ -675,16 +684,193 @@ __device__ __forceinline__ void fa_fwd_body(const FaArgs& p) {
   }
 }
 
+// Few or short heads: a workgroup owns 32 queries of one (batch, head), and its four waves take
+// every fourth key tile of them, each through its own pipeline (no barriers) with the tile and
+// probability code of FaState, then add up their parts relative to a common reference point.
+// Bound by the chain of tiles each wave goes through (about 0.8 us a tile at head_dim 64, 1.5 at
+// 128, one wave per SIMD): the chain is a quarter of the sequence, and four (head_dim 64) or eight
+// times as many workgroups as fa_fwd_body's spread over the CUs.  In exchange K and V are read
+// once per 32 queries.  fa_fwd_body, here (us, non-causal): 2x8 heads, 777 keys, head_dim 64: 13.8,
+// 10.2; 8 heads, 1024 keys, head_dim 128: 27.6, 12.6; 1 head, 4096 keys: 86.5, 28.9.
+// (Two query blocks per wave, QB = 2, halve the reads but double the chain's MFMAs: 18.8 us for
+// the 8 heads, and at most 15% faster where the launch fills the chip twice, where
+// fa_fwd_body is the better one in most cases.)
+template <int D>
+struct FaSplit {
+  static constexpr int kWaves = 4, QB = 1, kWgPerCu = D == 64 ? 2 : 1;
+  static constexpr int kQueries = 32 * QB;  // per workgroup
+};
+
+template <int D>
+__device__ __forceinline__ void fa_split_body(const FaArgs& p) {
+  constexpr int QB = FaSplit<D>::QB;
+  using St = FaState<D, 1, QB>;
+  constexpr int kWaves = FaSplit<D>::kWaves;
+  constexpr int kTileBytes = St::kTileBytes;
+  constexpr int kKSteps = St::kKSteps, kDBlocks = St::kDBlocks;
+  constexpr int kLoads = St::kLoadsPerWave;
+  constexpr int BQ = FaSplit<D>::kQueries;
+  constexpr int kRow = D * 4;  // bytes of a query's row of partial results
+  static_assert(BQ * kRow <= 2 * kTileBytes, "a wave's partial results reuse its tiles");
+  // one K and one V tile per wave
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kWaves * 2 * kTileBytes];
+  __shared__ float stats[2][kWaves][BQ];  // reference point and sum of each wave and query
+
+  St st;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint8_t* ring = lds + wave * 2 * kTileBytes;
+  st.lane = tid & 63;
+  st.wave = 0;
+  st.col = st.lane & 31;
+  st.h = st.lane >> 5;
+  const int col = st.col, h = st.h;
+  int64_t bh;
+  int qblk;
+  fa_block(p, bh, qblk);
+  const int q0 = qblk * BQ;
+  const int S = p.seq;
+  const int64_t head_off = bh * static_cast<int64_t>(S) * D;
+  st.q0 = q0;
+  st.S = S;
+  st.causal = p.causal;
+  st.scale_log2 = p.scale_log2;
+  st.qw0 = q0;
+  st.init_loads(p.k + head_off, p.v + head_off);
+
+  const int kv_end = p.causal ? min(S, q0 + BQ) : S;
+  const int n_tiles = (kv_end + BKV - 1) / BKV;
+
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const int q = st.my_q(qb);
+#pragma unroll
+    for (int ks = 0; ks < kKSteps; ++ks) {
+      st.qreg[qb][ks] = u32x4{0, 0, 0, 0};
+      if (q < S) {
+        st.qreg[qb][ks] =
+            *reinterpret_cast<const u32x4*>(p.q + head_off + static_cast<int64_t>(q) * D + ks * 16 + h * 8);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kDBlocks; ++i) st.acc_o[qb][i] = f32x16{};
+    st.m_run[qb] = -INFINITY;
+    st.l_part[qb] = 0.f;
+  }
+
+  // K of the next tile is loaded while this tile's probabilities are taken and multiplied, V of
+  // the next tile during its scores: each into the stage whose last read has just been waited for.
+  uint8_t* vring = ring + kTileBytes;
+  if (wave < n_tiles) {
+    st.template load_tile<false>(ring, wave * BKV);
+    st.template load_tile<true>(vring, wave * BKV);
+  }
+  for (int j = wave; j < n_tiles; j += kWaves) {
+    const bool next = j + kWaves < n_tiles;
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");  // all but V_j have landed
+    f32x16 s[QB][2];
+    st.scores(ring, s);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (next) st.template load_tile<false>(ring, (j + kWaves) * BKV);
+    st.mask(s, j * BKV);
+    u32x4 pb[QB][2][2];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      if (j == wave) st.raise(qb, st.tile_max(s[qb]));
+      float rs = st.probs(qb, s[qb], pb[qb]);
+      if (__builtin_amdgcn_ballot_w64(rs > kTileSumLimit) != 0) {
+        st.raise(qb, st.tile_max(s[qb]));
+        rs = st.probs(qb, s[qb], pb[qb]);
+      }
+      st.l_part[qb] += rs;
+    }
+    if (next) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");  // all but K of the next tile
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    st.pv(vring, pb);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (next) st.template load_tile<true>(vring, (j + kWaves) * BKV);
+  }
+
+  // The parts: O^T of a wave relative to its own reference point, transposed through LDS.
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  // 16-byte chunk c of a row at c ^ (row % 16): 16 rows' writes of one chunk hit all banks
+  const auto part_off = [](int row, int c) { return row * kRow + ((c ^ (row & 15)) << 4); };
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    const int row = qb * 32 + col;
+    const float l = st.l_part[qb] + other_half(st.l_part[qb]);
+    if (h == 0) {
+      stats[0][wave][row] = st.m_run[qb];
+      stats[1][wave][row] = l;
+    }
+#pragma unroll
+    for (int db = 0; db < kDBlocks; ++db) {
+#pragma unroll
+      for (int rq = 0; rq < 4; ++rq) {
+        const f32x16& a = st.acc_o[qb][db];
+        *reinterpret_cast<f32x4*>(ring + part_off(row, db * 8 + rq * 2 + h)) =
+            f32x4{a[rq * 4], a[rq * 4 + 1], a[rq * 4 + 2], a[rq * 4 + 3]};
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < BQ * (D / 8) / (kWaves * 64); ++i) {
+    const int cc = tid + kWaves * 64 * i;
+    const int row = cc / (D / 8), ch = cc % (D / 8);
+    float m = stats[0][0][row];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) m = fmaxf(m, stats[0][w][row]);
+    float f[kWaves], l_run = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const float mw = stats[0][w][row];
+      f[w] = mw == m ? 1.0f : __builtin_amdgcn_exp2f(mw - m);
+      l_run += f[w] * stats[1][w][row];
+    }
+    const float inv_l = l_run > 0.f ? 1.0f / l_run : 0.f;
+    float o[8] = {};
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const uint8_t* part = lds + w * 2 * kTileBytes;
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(part + part_off(row, 2 * ch));
+      const f32x4 hi = *reinterpret_cast<const f32x4*>(part + part_off(row, 2 * ch + 1));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o[e] = fmaf(f[w], lo[e], o[e]);
+        o[4 + e] = fmaf(f[w], hi[e], o[4 + e]);
+      }
+    }
+    if (q0 + row < S) {
+      u32x4 w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = pack_bf16(o[2 * e] * inv_l, o[2 * e + 1] * inv_l);
+      *reinterpret_cast<u32x4*>(p.o + head_off + static_cast<int64_t>(q0 + row) * D + ch * 8) = w;
+      if (p.lse != nullptr && ch == 0) p.lse[bh * S + q0 + row] = (m + __log2f(l_run)) * 0.69314718055994530942f;
+    }
+  }
+}
+
 }  // namespace fa
 }  // namespace asc
 
-// Defines the attention kernels as PREFIX##d64 / PREFIX##d128 (head_dim 64 / 128),
-// each taking one asc::fa::FaArgs by value, with the given linkage specifier.
+// Defines the attention kernels as PREFIX##d64 / PREFIX##d128 (head_dim 64 / 128) and, with the
+// keys split over waves, PREFIX##d64_split / PREFIX##d128_split, each taking one asc::fa::FaArgs by value, with the given linkage specifier.
 #define ASC_FA_KERNEL(LINKAGE, NAME, D)                                                                            \
   LINKAGE __global__ void __launch_bounds__(asc::fa::FaConfig<D>::kWaves * 64, asc::fa::FaConfig<D>::kWgPerCu)    \
       NAME(asc::fa::FaArgs p) {                                                                                    \
     asc::fa::fa_fwd_body<D>(p);                                                                                    \
   }
-#define ASC_FA_KERNELS(LINKAGE, PREFIX) \
-  ASC_FA_KERNEL(LINKAGE, PREFIX##d64, 64)  \
-  ASC_FA_KERNEL(LINKAGE, PREFIX##d128, 128)
+#define ASC_FA_SPLIT_KERNEL(LINKAGE, NAME, D)                                                                      \
+  LINKAGE __global__ void __launch_bounds__(asc::fa::FaSplit<D>::kWaves * 64, asc::fa::FaSplit<D>::kWgPerCu)      \
+      NAME(asc::fa::FaArgs p) {                                                                                    \
+    asc::fa::fa_split_body<D>(p);                                                                                  \
+  }
+#define ASC_FA_KERNELS(LINKAGE, PREFIX)               \
+  ASC_FA_KERNEL(LINKAGE, PREFIX##d64, 64)             \
+  ASC_FA_KERNEL(LINKAGE, PREFIX##d128, 128)           \
+  ASC_FA_SPLIT_KERNEL(LINKAGE, PREFIX##d64_split, 64) \
+  ASC_FA_SPLIT_KERNEL(LINKAGE, PREFIX##d128_split, 128)

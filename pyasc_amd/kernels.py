@@ -533,10 +533,21 @@ def flash_attention_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: to
 
 def flash_attention_plan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, sm_scale: float,
                          causal: bool, lse: Optional[torch.Tensor] = None) -> "_native.LaunchPlan":
-    """The launch flash_attention_fwd(...) makes, as a kernel of the asc2_flash_attention
-    code object with its grid, block and argument blob (asc_flash_attention_plan)."""
+    """A launch of flash_attention_fwd(...) without a split of the keys, as a kernel of the
+    asc2_flash_attention code object with its grid, block and argument blob
+    (asc_flash_attention_plan)."""
     plan = _native.LaunchPlan()
     _native.call("asc_flash_attention_plan", *_attention_args(q, k, v, o, sm_scale, causal, lse),
+                 ctypes.byref(plan))
+    return plan
+
+
+def flash_attention_dispatch(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, sm_scale: float,
+                             causal: bool, lse: Optional[torch.Tensor] = None) -> "_native.LaunchPlan":
+    """The launch flash_attention_fwd(...) makes (asc_flash_attention_dispatch), in
+    flash_attention_plan's form."""
+    plan = _native.LaunchPlan()
+    _native.call("asc_flash_attention_dispatch", *_attention_args(q, k, v, o, sm_scale, causal, lse),
                  ctypes.byref(plan))
     return plan
 

@@ -527,11 +527,12 @@ def _attention_views(call: KernelCall):
 
 def _attention_code_object_launch(call: KernelCall, functions) -> None:
     q, k, v, o = _attention_views(call)
-    module.launch_plan(functions, kernels.flash_attention_plan(q, k, v, o, float(call.get("sm_scale")),
-                                                               bool(call.get("causal"))), call.stream)
+    module.launch_plan(functions, kernels.flash_attention_dispatch(q, k, v, o, float(call.get("sm_scale")),
+                                                                   bool(call.get("causal"))), call.stream)
 
 
-ATTENTION_CODE_OBJECT = module.CodeObject("asc2_flash_attention", ("asc2_fa_fwd_d64", "asc2_fa_fwd_d128"),
+ATTENTION_CODE_OBJECT = module.CodeObject("asc2_flash_attention", ("asc2_fa_fwd_d64", "asc2_fa_fwd_d128",
+                                                                   "asc2_fa_fwd_d64_split", "asc2_fa_fwd_d128_split"),
                                           _attention_code_object_launch,
                                           "pyasc_amd/csrc/co/asc2_flash_attention.hip")
 
