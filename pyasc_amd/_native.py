@@ -147,14 +147,23 @@ def load_library(path: Optional[Path] = None) -> ctypes.CDLL:
         return lib
 
 
+_torch_c = None  # torch._C once the device is initialised and it has the calls used below
+
+
 def current_stream_handle() -> int:
     """hipStream_t of torch's current stream on the current device, read without building
     a torch Stream object (the launch paths ask for it on every call)."""
+    global _torch_c
+    c = _torch_c
+    if c is not None and not c._cuda_isInBadFork():
+        return c._cuda_getCurrentRawStream(c._cuda_getDevice())
     import torch
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if raw is None:
+    if getattr(torch._C, "_cuda_getCurrentRawStream", None) is None:
         return int(torch.cuda.current_stream().cuda_stream)
-    return int(raw(torch.cuda.current_device()))
+    handle = int(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+    if hasattr(torch._C, "_cuda_getDevice") and hasattr(torch._C, "_cuda_isInBadFork"):
+        _torch_c = torch._C
+    return handle
 
 
 def last_error() -> str:
@@ -170,8 +179,9 @@ def check(code: int, fn_name: str) -> None:
 
 
 def call(fn_name: str, *args) -> None:
-    fn = getattr(load_library(), fn_name)
-    check(fn(*args), fn_name)
+    code = getattr(_lib or load_library(), fn_name)(*args)
+    if code != 0:
+        check(code, fn_name)
 
 
 def version() -> str:

@@ -20,6 +20,7 @@ cache, as it bypasses the reference's.
 """
 from __future__ import annotations
 
+import functools
 import hashlib
 import inspect
 import re
@@ -43,6 +44,11 @@ _CONFIG_KEYWORDS = frozenset(CODEGEN_OPTIONS + COMPILE_OPTIONS + LAUNCH_OPTIONS)
 
 
 _UNSET = object()
+
+
+@functools.lru_cache(maxsize=256)
+def _grid_options(core_num: int) -> LaunchOptions:
+    return LaunchOptions(core_num=core_num)
 
 
 class ArgType:
@@ -122,7 +128,9 @@ class JITFunction:
 
     def __getitem__(self, user_launch_options: Union[int, tuple]) -> Callable:
         try:
-            if isinstance(user_launch_options, int):
+            if user_launch_options.__class__ is int:
+                self.launch_options = _grid_options(user_launch_options)
+            elif isinstance(user_launch_options, int):
                 self.launch_options = LaunchOptions(core_num=user_launch_options)
             else:
                 self.launch_options = LaunchOptions(*user_launch_options)
@@ -290,14 +298,14 @@ class JITFunction:
             if cls is int or cls is float or cls is bool:
                 parts.append(cls)
             elif cls.__module__ == "torch" and cls.__name__ in ("Tensor", "Parameter"):
-                parts.append((value.dtype, value.dim() == 0))
+                parts.append(value.dtype)
+                parts.append(value.dim() == 0)
             else:
                 return None
         try:
-            consts = tuple(_tagged(v) for v in constexprs.values())
-            opts = tuple(sorted((k, _tagged(v)) for k, v in call_options.items() if k not in LAUNCH_OPTIONS)) \
-                if call_options else ()
-            key = (tuple(parts), consts, opts)
+            key = (tuple(parts), tuple([_tagged(v) for v in constexprs.values()]),
+                   tuple(sorted((k, _tagged(v)) for k, v in call_options.items() if k not in LAUNCH_OPTIONS))
+                   if call_options else ())
             hash(key)
         except TypeError:
             return None
@@ -337,7 +345,9 @@ class JITFunction:
 
     def _run(self, *args, **kwargs) -> None:
         resolved, runtime_args, constexprs = self.resolve(*args, **kwargs)
-        options = {**self.default_options, **{k: v for k, v in kwargs.items() if k in COMPILE_OPTIONS}}
+        options = self.default_options
+        if kwargs:
+            options = {**options, **{k: v for k, v in kwargs.items() if k in COMPILE_OPTIONS}}
         Launcher(self.launch_options).run(resolved.entry, self.fn_name, runtime_args, constexprs, options,
                                           resolved=resolved if resolved.cache_key else None)
 

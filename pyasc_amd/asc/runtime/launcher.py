@@ -102,7 +102,11 @@ class Launcher:
         device_args: Dict[str, Any] = {}
         copy_back: List[Tuple[Any, Any]] = []
         for name, value in runtime_args.items():
-            if isinstance(value, np.ndarray):
+            cls = value.__class__
+            if cls is int or cls is float or cls is bool or (cls is torch.Tensor and value.is_cuda and
+                                                             value.is_contiguous() and value.dim() > 0):
+                device_args[name] = value  # most arguments: nothing to convert
+            elif isinstance(value, np.ndarray):
                 dev = torch.from_numpy(np.ascontiguousarray(value)).to("cuda")
                 device_args[name] = dev
                 copy_back.append((value, dev))
@@ -137,7 +141,7 @@ class Launcher:
             if stream != _native.current_stream_handle():
                 torch.cuda.current_stream().synchronize()
         call = KernelCall(function_name, device_args, constexprs, int(self.options.core_num), stream,
-                          {"options": dict(options or {})})
+                          {"options": dict(options) if options else {}})
         if entry.code_object is None:
             entry.launch(call)
         else:

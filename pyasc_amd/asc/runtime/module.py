@@ -118,7 +118,8 @@ def _layout(kinds: Tuple[str, ...]) -> struct.Struct:
 def pack_args(fields: Sequence[Tuple[str, object]]) -> bytes:
     """Kernel arguments as one blob: each field ("ptr" / "i64" / "i32" / "f32", value)
     at its natural alignment, the way the kernel's argument list lays them out."""
-    return _layout(tuple(kind for kind, _ in fields)).pack(*(value for _, value in fields))
+    kinds, values = zip(*fields) if fields else ((), ())
+    return _layout(kinds).pack(*values)
 
 
 def launch(function: int, grid: int, block: int, fields: Sequence[Tuple[str, object]], stream: int) -> None:
@@ -132,8 +133,7 @@ def launch_blob(function: int, grid: int, block: int, blob: bytes, stream: int) 
     kernel declares its arguments."""
     if grid <= 0 or block <= 0 or grid * block >= 1 << 32:
         raise ValueError(f"{grid} workgroups of {block} threads: outside the launch range (under 2^32 threads)")
-    buf = ctypes.create_string_buffer(blob, len(blob))
-    _native.call("asc_module_launch", ctypes.c_void_p(function), grid, block, buf, len(blob), ctypes.c_void_p(stream))
+    _native.call("asc_module_launch", function, grid, block, blob, len(blob), stream)
     stats["launches"] += 1
 
 

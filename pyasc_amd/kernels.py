@@ -35,7 +35,7 @@ def _stream(stream: Any) -> int:
 def _device_tensor(t: Any, name: str) -> torch.Tensor:
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"'{name}' must be a torch.Tensor, got {type(t).__name__}")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"'{name}' must be on the HIP device, got {t.device}")
     return t
 
@@ -67,13 +67,15 @@ def vadd_covered(size: int, tile_size: int, tile_per_block: int, grid: int) -> i
     return max(0, min(size, grid * tile_per_block * tile_size))
 
 
+_VADD_DTYPES = (torch.float32, torch.float16, torch.bfloat16, torch.int32)
+
+
 def vadd_check(x: torch.Tensor, y: torch.Tensor, out: torch.Tensor, size: int, tile_size: int, tile_per_block: int,
                grid: int) -> int:
     """Host checks of a vadd launch; returns the covered element count."""
     for t, n in ((x, "x"), (y, "y"), (out, "out")):
         _contiguous(_device_tensor(t, n), n)
-    allowed = (torch.float32, torch.float16, torch.bfloat16, torch.int32)
-    _code(x, "x", allowed)
+    _code(x, "x", _VADD_DTYPES)
     if y.dtype != x.dtype or out.dtype != x.dtype:
         raise TypeError(f"vadd operands must share one dtype, got {x.dtype}, {y.dtype}, {out.dtype}")
     if tile_size <= 0 or tile_per_block < 0 or grid <= 0 or size < 0:

@@ -61,10 +61,11 @@ def _stream_code_object(functions, vec: str, elem: str, tensors, covered: int, e
     object: kernel ``vec`` over the 16-byte vectors of [0, covered) when every tensor is
     16-byte aligned, kernel ``elem`` over the rest; the kernels take the tensors'
     pointers, then the range, then ``extra``."""
-    ptrs = [("ptr", t.data_ptr()) for t in tensors]
+    addrs = [t.data_ptr() for t in tensors]
+    ptrs = [("ptr", a) for a in addrs]
     per_vec = 16 // tensors[0].element_size()
     done = 0
-    if all(t.data_ptr() % 16 == 0 for t in tensors):
+    if all([a % 16 == 0 for a in addrs]):
         n_vec = covered // per_vec
         if n_vec:
             module.launch(functions[vec], ceildiv(n_vec, STREAM_THREADS * STREAM_UNROLL), STREAM_THREADS,
