@@ -203,7 +203,7 @@ int32_t asc_softmax_blocks_f32(const float* x, float* out, int64_t num_rows,
 /* The same two kernels on float16 x / out (asc2.softmax on an f16 tile,
  * which the op allows: python/asc/language/tile/unary_ops.py:213-222;
  * python/test/asc2/operations/test_softmax.py).  fp32 statistics (x - max in
- * fp32, libm exp, one reciprocal of the sum), each output rounded once (RNE)
+ * fp32, exp to about 2 ulp, one reciprocal of the sum), each output rounded once (RNE)
  * to float16.  Same coverage rules as the float32 entries. */
 int32_t asc_softmax_rows_f16(const void* x, void* out, int64_t num_rows,
                              int64_t num_cols, int32_t tile_size, int32_t grid,
@@ -235,9 +235,10 @@ typedef struct asc_softmax_plan {
 int32_t asc_softmax_plan(int32_t dtype, int32_t fused, const void* x,
                          const void* out, int64_t num_rows, int64_t num_cols,
                          int32_t size, int32_t grid, asc_softmax_plan_t* plan);
-/* The launch the four entries make: asc_softmax_plan's, or for few or long rows
- * the same softmax with 1024 threads per row, and for short float16 rows a grid
- * of no more workgroups than the rows need.  Same arguments and errors. */
+/* The launch the four entries make: asc_softmax_plan's, or the same softmax with
+ * 1024 threads per row for long rows and 16 lanes per row for many short float32
+ * rows, and for float16 a grid of no more workgroups than the rows need.  Same
+ * arguments and errors. */
 int32_t asc_softmax_dispatch(int32_t dtype, int32_t fused, const void* x,
                              const void* out, int64_t num_rows,
                              int64_t num_cols, int32_t size, int32_t grid,
@@ -417,7 +418,7 @@ int32_t asc_flash_attention_fwd_bf16(const void* q, const void* k,
                                      int64_t seq_len, int32_t head_dim,
                                      float sm_scale, int32_t causal,
                                      asc_stream_t stream);
-/* The launch asc_flash_attention_fwd_bf16 makes with these arguments, as a
+/* The launch of asc_flash_attention_fwd_bf16 without a split of the keys, as a
  * kernel of the code object pyasc_amd/lib/co/asc2_flash_attention.hsaco.  Same
  * checks and errors (a causal plan reads the current device's CU count). */
 int32_t asc_flash_attention_plan(const void* q, const void* k, const void* v,

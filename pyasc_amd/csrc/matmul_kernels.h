@@ -5,6 +5,10 @@
 // (python/asc/language/tile/binary_ops.py:180-221; kernels in
 // python/test/asc2/kernels/test_matmul_{mnblock,tiled,fixpipe,l0c_to_l1}.py).
 //
+// These are the kernels of large products (and of asc_matmul_plan); small, ragged and
+// unaligned ones run on gemm_tile.h's where those are the better ones
+// (asc_matmul_dispatch, matmul_tile.h).
+//
 // fp16/bf16 inputs run on MFMA (v_mfma_f32_32x32x16_{bf16,f16}) with fp32
 // accumulation and a 256x256 output tile per workgroup:
 //   - tile-aligned shapes (M, N multiples of 256, K of 32, offsets within

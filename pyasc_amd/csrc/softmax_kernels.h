@@ -15,9 +15,9 @@
 // bodies (which load and store at element alignment and do not need it) and the
 // pad count (tile - num_cols) for the padded bodies.
 //
-// HBM-bound (one read + one write of every element).  Rows up to 8192 columns
-// stay in registers: a wave per row (two rows per wave) up to 512 columns, a
-// 128- or 256-thread block per row above (asc_softmax_plan picks the body).  Max,
+// HBM-bound (one read + one write of every element).  Rows up to 49152 fp32 or 65529
+// fp16 columns stay in registers: 16 lanes, a wave or a workgroup per row, by its
+// length and the number of rows (asc_softmax_dispatch picks the body).  Max,
 // min and sum reduce in-thread, then across the wave with DPP and permlane
 // swaps (no LDS round trips), then across waves through LDS.  x - max is
 // rounded to fp32 as in the reference (test_softmax.py:22-24); exp of it is
