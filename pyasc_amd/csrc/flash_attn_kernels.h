@@ -857,8 +857,9 @@ __device__ __forceinline__ void fa_split_body(const FaArgs& p) {
 }  // namespace fa
 }  // namespace asc
 
-// Defines the attention kernels as PREFIX##d64 / PREFIX##d128 (head_dim 64 / 128) and, with the
-// keys split over waves, PREFIX##d64_split / PREFIX##d128_split, each taking one asc::fa::FaArgs by value, with the given linkage specifier.
+// Defines the attention kernels as PREFIX##d64 / PREFIX##d128 (head_dim 64 / 128) and, with
+// the keys split over waves, PREFIX##d64_split / PREFIX##d128_split, each taking one
+// asc::fa::FaArgs by value, with the given linkage specifier.
 #define ASC_FA_KERNEL(LINKAGE, NAME, D)                                                                            \
   LINKAGE __global__ void __launch_bounds__(asc::fa::FaConfig<D>::kWaves * 64, asc::fa::FaConfig<D>::kWgPerCu)    \
       NAME(asc::fa::FaArgs p) {                                                                                    \

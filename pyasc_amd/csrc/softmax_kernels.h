@@ -416,13 +416,13 @@ __device__ __forceinline__ void wide_body(const void* x, void* out, int64_t rows
 // to about 2 ulp, one reciprocal of the sum, then one RNE rounding of each output to fp16.
 // A row belongs to 16 lanes (up to 505 columns), a wave (up to 4089), a workgroup of 256
 // threads (up to 16377) or one of 1024, and stays in registers as fp32, up to 64 values per
-// thread, so x is read once; past 65529 columns it is read twice.  A row starts on any half, and 16-byte accesses at odd halves
-// run at half rate, so vectors are aligned in memory, not to the row: vector q holds the
-// row's elements 8q - h .. 8q - h + 7, h the halves between the row and the aligned address
-// before it, and elements outside the row become -inf.  HBM-bound (4 B per element); a
-// workgroup per row and separate passes for maximum, sum and result before, here (us):
-// 3000x10007 87.6, 25.9; 4096x4096 23.6, 16.8; 100000x64 117, 12.4; 30000x1000 62, 25;
-// 11926x2314 78, 25; 2000x32000 101, 63; 640x100003 385, 95.
+// thread, so x is read once; past 65529 columns it is read twice.  A row starts on any half,
+// and 16-byte accesses at odd halves run at half rate, so vectors are aligned in memory, not
+// to the row: vector q holds the row's elements 8q - h .. 8q - h + 7, h the halves between the
+// row and the aligned address before it, and elements outside the row become -inf.  HBM-bound
+// (4 B per element); a workgroup per row and separate passes for maximum, sum and result
+// before, here (us): 3000x10007 87.6, 25.9; 4096x4096 23.6, 16.8; 100000x64 117, 12.4;
+// 30000x1000 62, 25; 11926x2314 78, 25; 2000x32000 101, 63; 640x100003 385, 95.
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
 
