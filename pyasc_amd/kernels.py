@@ -40,11 +40,17 @@ def _device_tensor(t: Any, name: str) -> torch.Tensor:
     return t
 
 
-def _keep_for_stream(workspace: torch.Tensor, handle: int) -> None:
-    """A workspace is freed when its call returns: on a stream other than torch's current one
-    the caching allocator must not hand its memory out again before the launches have run."""
-    if handle != torch.cuda.current_stream(workspace.device).cuda_stream:
-        workspace.record_stream(torch.cuda.ExternalStream(handle, device=workspace.device))
+def workspace_on(handle: int, numel: int, dtype: torch.dtype, device: torch.device) -> torch.Tensor:
+    """A workspace for the launches of one call on stream ``handle``, freed when the call returns.
+    It comes from that stream's pool of torch's allocator: a block of another stream's pool may
+    still be in use by work queued there, and would be handed out again before the launches have
+    run, while a block of the launch stream's pool is ordered with them on both sides."""
+    if handle == torch.cuda.current_stream(device).cuda_stream:
+        return torch.empty(numel, dtype=dtype, device=device)
+    # handle 0 is the default stream, which an ExternalStream cannot name
+    stream = torch.cuda.ExternalStream(handle, device=device) if handle else torch.cuda.default_stream(device)
+    with torch.cuda.stream(stream):
+        return torch.empty(numel, dtype=dtype, device=device)
 
 
 def _contiguous(t: torch.Tensor, name: str) -> torch.Tensor:
@@ -291,7 +297,7 @@ _REDUCE_SPLIT_MIN = 1 << 18
 
 def _reduce(x: torch.Tensor, out: torch.Tensor, op: str, rows: int, cols: int, dim: int, count: int, stream) -> None:
     """One reduction; one with few results over many elements gets a workspace (at most 64 KiB)
-    from torch's allocator on the launch stream for its partial results."""
+    for its partial results, from the launch stream's pool of torch's allocator."""
     handle = _stream(stream)
     args = (REDUCE_OPS[op], x.data_ptr(), out.data_ptr(), rows, cols, dim, count)
     nbytes = 0
@@ -300,8 +306,7 @@ def _reduce(x: torch.Tensor, out: torch.Tensor, op: str, rows: int, cols: int, d
     if nbytes == 0:
         _native.call("asc_reduce_f32", *args, handle)
         return
-    workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    _keep_for_stream(workspace, handle)
+    workspace = workspace_on(handle, nbytes, torch.uint8, x.device)
     _native.call("asc_reduce_f32_ws", *args, workspace.data_ptr(), nbytes, handle)
 
 
@@ -395,7 +400,7 @@ def matmul_chained(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, workspace:
     """The asc2 chained matmul (python/test/asc2/kernels/test_matmul_l0c_to_l1.py:17-30):
     t = (a @ b) cast to a's dtype, c = cast(t @ b) to c's dtype, fp32 accumulation, N == K.
     ``workspace`` (a contiguous device tensor of at least M * N * 2 bytes) holds t; without
-    one it is taken from torch's allocator on the launch stream."""
+    one it is taken from the launch stream's pool of torch's allocator."""
     for t, n in ((a, "a"), (b, "b"), (c, "c")):
         _contiguous(_device_tensor(t, n), n)
     in_code = _code(a, "a", (torch.float16, torch.bfloat16))
@@ -413,8 +418,7 @@ def matmul_chained(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, workspace:
         raise ValueError(f"c must be {(M, N)}, got {tuple(c.shape)}")
     handle = _stream(stream)
     if workspace is None:
-        workspace = torch.empty(M * N, dtype=a.dtype, device=a.device)
-        _keep_for_stream(workspace, handle)
+        workspace = workspace_on(handle, M * N, a.dtype, a.device)
     else:
         _contiguous(_device_tensor(workspace, "workspace"), "workspace")
     nbytes = workspace.numel() * workspace.element_size()

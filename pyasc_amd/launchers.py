@@ -395,13 +395,9 @@ def _chained_body(call: KernelCall, mm, chained=None) -> None:
     if chained is not None and a.dtype in (torch.float16, torch.bfloat16):
         chained(a, b, c, stream=call.stream)
         return
-    t = torch.empty((M, N), dtype=mid_dtype, device=a.device)
+    t = kernels.workspace_on(call.stream, M * N, mid_dtype, a.device).view(M, N)
     mm(a, b, t, stream=call.stream)
     mm(t, b, c, stream=call.stream)
-    # t is freed on return; on a stream other than torch's current one the caching
-    # allocator must not hand its memory out again before these launches have run
-    if call.stream != torch.cuda.current_stream(a.device).cuda_stream:
-        t.record_stream(torch.cuda.ExternalStream(call.stream, device=a.device))
 
 
 # The tile kernels of csrc/matmul_tile.h: fp16 / bf16 / int8, and fp32.
