@@ -53,6 +53,27 @@ def workspace_on(handle: int, numel: int, dtype: torch.dtype, device: torch.devi
         return torch.empty(numel, dtype=dtype, device=device)
 
 
+def _capturing(handle: int, device: torch.device) -> bool:
+    """Whether stream ``handle`` is recording a graph."""
+    if handle == torch.cuda.current_stream(device).cuda_stream:
+        return torch.cuda.is_current_stream_capturing()
+    if handle == 0:
+        return False  # the default stream cannot be captured
+    with torch.cuda.stream(torch.cuda.ExternalStream(handle, device=device)):
+        return torch.cuda.is_current_stream_capturing()
+
+
+def _held_by_a_graph(t: torch.Tensor) -> bool:
+    """Whether ``t``, allocated during a capture, lies in a graph's own memory pool: torch keeps
+    that for the graph's replays.  In a capture begun by other means the block is an ordinary
+    one, which goes to the next allocation once it is freed."""
+    if torch.cuda.get_allocator_backend() != "native":
+        return False
+    at = t.data_ptr()
+    return any(s["address"] <= at < s["address"] + s["total_size"] and s.get("segment_pool_id", (0, 0)) != (0, 0)
+               for s in torch.cuda.memory_snapshot())
+
+
 def _contiguous(t: torch.Tensor, name: str) -> torch.Tensor:
     if not t.is_contiguous():
         raise ValueError(f"'{name}' must be contiguous")
@@ -297,7 +318,9 @@ _REDUCE_SPLIT_MIN = 1 << 18
 
 def _reduce(x: torch.Tensor, out: torch.Tensor, op: str, rows: int, cols: int, dim: int, count: int, stream) -> None:
     """One reduction; one with few results over many elements gets a workspace (at most 64 KiB)
-    for its partial results, from the launch stream's pool of torch's allocator."""
+    for its partial results, from the launch stream's pool of torch's allocator.  Under a capture
+    that torch does not know of, whose replays would find that workspace given to others, it
+    runs without one."""
     handle = _stream(stream)
     args = (REDUCE_OPS[op], x.data_ptr(), out.data_ptr(), rows, cols, dim, count)
     nbytes = 0
@@ -307,6 +330,9 @@ def _reduce(x: torch.Tensor, out: torch.Tensor, op: str, rows: int, cols: int, d
         _native.call("asc_reduce_f32", *args, handle)
         return
     workspace = workspace_on(handle, nbytes, torch.uint8, x.device)
+    if _capturing(handle, x.device) and not _held_by_a_graph(workspace):
+        _native.call("asc_reduce_f32", *args, handle)
+        return
     _native.call("asc_reduce_f32_ws", *args, workspace.data_ptr(), nbytes, handle)
 
 

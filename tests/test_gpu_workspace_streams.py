@@ -1,6 +1,8 @@
 """Workspaces of launches on another stream than torch's current one, while the current stream
 still has work queued on blocks that are already free again in its pool: the split reductions
 and the chained matmul must neither disturb that work nor be disturbed by it."""
+import ctypes
+
 import pytest
 import torch
 
@@ -63,3 +65,46 @@ def test_the_null_handle_is_the_default_stream(device):
     del w
     y = torch.empty(4096, dtype=torch.uint8, device=device)
     assert y.data_ptr() == ptr and x.data_ptr() != ptr
+
+
+def _hip():
+    """The HIP runtime that this process has loaded."""
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    hip = ctypes.CDLL(path)
+    hip.hipStreamBeginCapture.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    hip.hipStreamEndCapture.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p)]
+    hip.hipGraphInstantiate.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_void_p, ctypes.c_void_p,
+                                        ctypes.c_void_p, ctypes.c_size_t]
+    hip.hipGraphLaunch.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    hip.hipGraphExecDestroy.argtypes = hip.hipGraphDestroy.argtypes = [ctypes.c_void_p]
+    return hip
+
+
+@pytest.mark.parametrize("current", [True, False])
+def test_reduction_in_a_graph_captured_without_torch(device, current):
+    # the replays must not depend on memory that torch takes back when the call returns
+    hip, relaxed = _hip(), 2
+    x = torch.rand(16384, 100, device=device)
+    out, want = torch.empty(100, device=device), torch.empty(100, device=device)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph, executable = ctypes.c_void_p(), ctypes.c_void_p()
+    with torch.cuda.stream(s if current else torch.cuda.current_stream()):
+        assert hip.hipStreamBeginCapture(s.cuda_stream, relaxed) == 0
+        kernels.reduce_f32(x, out, "sum", 0, stream=None if current else s)
+        assert hip.hipStreamEndCapture(s.cuda_stream, ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(executable), graph, None, None, 0) == 0
+    for _ in range(3):
+        x.copy_(torch.rand(16384, 100, device=device))
+        kernels.reduce_f32(x, want, "sum", 0)
+        with torch.cuda.stream(s):  # whoever gets a workspace's memory next keeps it
+            others = [torch.full((n,), 3.0, device=device) for n in (12800, 16384, 1000)]
+        torch.cuda.synchronize()
+        assert hip.hipGraphLaunch(executable, s.cuda_stream) == 0
+        torch.cuda.synchronize()
+        # sums of 16384 non-negative values in two orders
+        assert ((out - want).abs() <= 2 * 16384 * 2.0 ** -24 * want).all()
+        assert all(bool((o == 3.0).all()) for o in others)
+        del others
+    assert hip.hipGraphExecDestroy(executable) == 0 and hip.hipGraphDestroy(graph) == 0

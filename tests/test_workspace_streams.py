@@ -33,6 +33,8 @@ def streams(monkeypatch):
     monkeypatch.setattr(torch.cuda, "ExternalStream", lambda ptr, device=None: SimpleNamespace(
         cuda_stream=ptr or 0xBAD))
     monkeypatch.setattr(torch.cuda, "stream", use)
+    state.capturing = set()
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state.current[-1] in state.capturing)
     monkeypatch.setattr(_native, "current_stream_handle", lambda: state.current[-1])
     real_empty = torch.empty
 
@@ -76,3 +78,21 @@ def test_chained_launch_intermediate(streams, handle):
     launchers._chained_body(call, lambda a, b, c, stream: seen.append((tuple(c.shape), stream)))
     assert seen == [((8, 16), handle)] * 2
     assert streams.allocated == [handle] and streams.current == [CURRENT]
+
+
+@pytest.mark.parametrize("stream,handle", [(None, CURRENT), (OTHER, OTHER)])
+@pytest.mark.parametrize("pool,entry", [((0, 0), "asc_reduce_f32"), ((1, 0), "asc_reduce_f32_ws"),
+                                        (None, "asc_reduce_f32")])
+def test_reduction_under_capture(streams, monkeypatch, stream, handle, pool, entry):
+    # a graph's replays outlive the call: only a workspace in the graph's own pool may be recorded
+    segment = {"address": 0, "total_size": 1 << 62}
+    monkeypatch.setattr(torch.cuda, "memory_snapshot", lambda: [
+        segment if pool is None else {**segment, "segment_pool_id": pool}])
+    monkeypatch.setattr(torch.cuda, "get_allocator_backend", lambda: "native")
+    x, out = torch.zeros(8192, 64), torch.zeros(64)
+    streams.capturing = {handle}
+    kernels.reduce_f32(x, out, "sum", 0, stream=stream)
+    streams.capturing = {CURRENT, OTHER} - {handle}  # another stream's capture is no concern
+    kernels.reduce_f32(x, out, "sum", 0, stream=stream)
+    assert streams.launched == [(entry, handle), ("asc_reduce_f32_ws", handle)]
+    assert streams.current == [CURRENT]
