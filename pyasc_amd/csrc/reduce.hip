@@ -22,6 +22,8 @@
 // from 1024 fp32 / 2048 fp16 columns up).
 #include <math.h>
 
+#include <type_traits>
+
 #include "common.h"
 #include "numeric.h"
 #include "rows.h"
@@ -35,8 +37,8 @@ __device__ __forceinline__ float identity() {
   return kOp == kSum ? 0.0f : kOp == kMax ? -INFINITY : kOp == kMin ? INFINITY : 1.0f;
 }
 
-template <int kOp>
-__device__ __forceinline__ float combine(float a, float b) {
+template <int kOp, class T>
+__device__ __forceinline__ T combine(T a, T b) {
   if constexpr (kOp == kSum) return a + b;
   if constexpr (kOp == kMax) return fmaxf(a, b);
   if constexpr (kOp == kMin) return fminf(a, b);
@@ -74,39 +76,69 @@ __device__ __forceinline__ f32x4_u load4(const float* p) {
 }
 
 // Elements [0, len) of x by the kThreads threads of a group (t: the thread's index in it):
-// kUnroll independent vector loads per lane in flight, in-lane partials combined in a fixed order.
-template <int kOp, int kThreads, int kUnroll>
-__device__ __forceinline__ float reduce_span(const float* x, int64_t len, int t) {
+// four independent vector loads per lane in flight, in-lane partials combined in a fixed order.
+// What is left, at most three vectors per thread, is loaded at once too, each into a chain of its
+// own; the up to three elements behind the last vector go to the thread after it, so that every
+// thread's share weighs about the same in the tree that follows.  The tests on what is left are
+// uniform first: a short row, one vector per lane or less, is bound by what it issues.
+template <int kOp, int kThreads, class Int>
+__device__ __forceinline__ float reduce_span(const float* x, Int len, int t) {
+  if (len <= kThreads) return t < len ? x[t] : identity<kOp>();
+  constexpr int kUnroll = 4;
   float acc[4] = {identity<kOp>(), identity<kOp>(), identity<kOp>(), identity<kOp>()};
-  const int64_t nvec = len / 4;
-  int64_t q = t;
-  for (; q + (kUnroll - 1) * kThreads < nvec; q += kUnroll * kThreads) {
+  const auto add4 = [&](int u, f32x4_u v) {
+    acc[u] = combine<kOp>(acc[u], combine<kOp>(combine<kOp>(v.x, v.y), combine<kOp>(v.z, v.w)));
+  };
+  const Int nvec = len / 4;
+  Int q0 = 0;  // vectors taken by the whole group
+  for (; q0 + kUnroll * kThreads <= nvec; q0 += kUnroll * kThreads) {
     f32x4_u v[kUnroll];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) v[u] = load4(x + 4 * (q + u * kThreads));
+    for (int u = 0; u < kUnroll; ++u) v[u] = load4(x + 4 * (q0 + t + u * kThreads));
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u)
-      acc[u % 4] = combine<kOp>(acc[u % 4], combine<kOp>(combine<kOp>(v[u].x, v[u].y), combine<kOp>(v[u].z, v[u].w)));
+    for (int u = 0; u < kUnroll; ++u) add4(u, v[u]);
   }
-  for (; q < nvec; q += kThreads) {
-    const f32x4_u v = load4(x + 4 * q);
-    acc[0] = combine<kOp>(acc[0], combine<kOp>(combine<kOp>(v.x, v.y), combine<kOp>(v.z, v.w)));
+  const int left = static_cast<int>(nvec - q0), rest = static_cast<int>(len - nvec * 4);
+  f32x4_u v[kUnroll];
+  float tail[3] = {identity<kOp>(), identity<kOp>(), identity<kOp>()};
+#pragma unroll
+  for (int u = 0; u < kUnroll; ++u) {
+    v[u] = f32x4_u{identity<kOp>(), identity<kOp>(), identity<kOp>(), identity<kOp>()};
+    if (left > u * kThreads && t + u * kThreads < left) v[u] = load4(x + 4 * (q0 + t + u * kThreads));
   }
-  if (nvec * 4 + t < len) acc[1] = combine<kOp>(acc[1], x[nvec * 4 + t]);  // at most 3 elements
+  if (rest > 0 && t == left % kThreads) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      if (i < rest) tail[i] = x[nvec * 4 + i];
+  }
+#pragma unroll
+  for (int u = 0; u < kUnroll; ++u)
+    if (left > u * kThreads) add4(u, v[u]);
+  if (rest > 0) acc[3] = combine<kOp>(acc[3], combine<kOp>(combine<kOp>(tail[0], tail[1]), tail[2]));
   return combine<kOp>(combine<kOp>(acc[0], acc[1]), combine<kOp>(acc[2], acc[3]));
 }
 
 // Combines one value per thread of a kThreads-thread workgroup; every thread gets the result.
+// The waves' sums are added in pairs, the last four in fp64: a chain of sixteen fp32 additions was
+// the largest part of a long row's rounding error (relative error against fp64, 300x65536: 6.0e-8
+// with the chain, 4.4e-8 with one wave per row, 2.9e-8 with all of them in fp64).
 template <int kOp, int kThreads>
 __device__ __forceinline__ float block_combine(float v) {
-  __shared__ float part[kThreads / 64];
+  constexpr int kWaves = kThreads / 64;
+  __shared__ float part[kWaves];
   v = wave_combine<kOp>(v);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
   __syncthreads();
-  float total = part[0];
+  float p[kWaves];
 #pragma unroll
-  for (int w = 1; w < kThreads / 64; ++w) total = combine<kOp>(total, part[w]);
-  return total;
+  for (int w = 0; w < kWaves; ++w) p[w] = part[w];
+#pragma unroll
+  for (int n = kWaves / 2; n >= 4; n /= 2)
+#pragma unroll
+    for (int w = 0; w < n; ++w) p[w] = combine<kOp>(p[w], p[w + n]);
+  using Part = std::conditional_t<kOp == kSum, double, float>;
+  const Part lo = combine<kOp, Part>(p[0], p[1]), hi = combine<kOp, Part>(p[2], p[3]);
+  return static_cast<float>(combine<kOp>(lo, hi));
 }
 
 // dim 1, a wave per row: rows 4*blockIdx.x + wave.
@@ -114,7 +146,8 @@ template <int kOp>
 __global__ void __launch_bounds__(256) reduce_rows_kernel(ReduceArgs p) {
   const int64_t r = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (r >= p.rows) return;
-  const float total = wave_combine<kOp>(reduce_span<kOp, 64, 4>(p.x + r * p.cols, p.cols, threadIdx.x & 63));
+  const int len = static_cast<int>(p.cols);
+  const float total = wave_combine<kOp>(reduce_span<kOp, 64>(p.x + r * p.cols, len, threadIdx.x & 63));
   if ((threadIdx.x & 63) == 0) p.out[r] = total;
 }
 
@@ -122,7 +155,8 @@ __global__ void __launch_bounds__(256) reduce_rows_kernel(ReduceArgs p) {
 template <int kOp>
 __global__ void __launch_bounds__(1024) reduce_long_rows_kernel(ReduceArgs p) {
   const int64_t r = blockIdx.x;
-  const float total = block_combine<kOp, 1024>(reduce_span<kOp, 1024, 4>(p.x + r * p.cols, p.cols, threadIdx.x));
+  const int len = static_cast<int>(p.cols);
+  const float total = block_combine<kOp, 1024>(reduce_span<kOp, 1024>(p.x + r * p.cols, len, threadIdx.x));
   if (threadIdx.x == 0) p.out[r] = total;
 }
 
@@ -224,7 +258,7 @@ template <int kOp>
 __global__ void __launch_bounds__(1024) reduce_all_kernel(ReduceArgs p) {
   const int64_t n = p.rows * p.cols;
   const int64_t e0 = span_start(n, blockIdx.x, gridDim.x), e1 = span_start(n, blockIdx.x + 1, gridDim.x);
-  const float total = block_combine<kOp, 1024>(reduce_span<kOp, 1024, 4>(p.x + e0, e1 - e0, threadIdx.x));
+  const float total = block_combine<kOp, 1024>(reduce_span<kOp, 1024>(p.x + e0, e1 - e0, threadIdx.x));
   if (gridDim.x > 1) {
     if (threadIdx.x == 0) p.out[blockIdx.x] = total;
     return;

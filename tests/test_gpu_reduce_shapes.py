@@ -91,3 +91,16 @@ def test_split_reduction_on_a_side_stream_and_in_a_graph(device):
         kernels.reduce_f32(x, want, "sum", 0)
         torch.cuda.synchronize()
         assert torch.equal(out, want), k
+
+
+@pytest.mark.parametrize("rows,cols", [(512, 65536), (512, 3000), (300, 100003), (1024, 4096)])
+def test_row_sums_round_like_a_binary_tree(device, rows, cols):
+    # the last additions of a sum carry its rounding error: in a binary tree their variances are
+    # 1 + 1/2 + 1/4 + ... < 2 times that of one rounding, (2^-24)^2 / 3 relative at most.  A chain
+    # over the parts of a row has 1 + (15/16)^2 + (14/16)^2 + ...
+    x = torch.rand(rows, cols, generator=torch.Generator(device=device).manual_seed(cols), device=device)
+    out = torch.empty(rows, device=device)
+    kernels.reduce_f32(x, out, "sum", 1)
+    ref = x.double().sum(1)
+    rms = ((out.double() - ref) / ref).square().mean().sqrt().item()
+    assert rms <= 2.0 ** -24 * (2 / 3) ** 0.5, rms
