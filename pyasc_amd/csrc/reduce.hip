@@ -33,7 +33,7 @@ namespace {
 enum ReduceOp { kSum = 0, kMax = 1, kMin = 2, kProd = 3 };
 
 template <int kOp>
-__device__ __forceinline__ float identity() {
+__host__ __device__ constexpr float identity() {
   return kOp == kSum ? 0.0f : kOp == kMax ? -INFINITY : kOp == kMin ? INFINITY : 1.0f;
 }
 
@@ -77,15 +77,21 @@ __device__ __forceinline__ f32x4_u load4(const float* p) {
 
 // Elements [0, len) of x by the kThreads threads of a group (t: the thread's index in it):
 // four independent vector loads per lane in flight, in-lane partials combined in a fixed order.
-// What is left, at most three vectors per thread, is loaded at once too, each into a chain of its
-// own; the up to three elements behind the last vector go to the thread after it, so that every
-// thread's share weighs about the same in the tree that follows.  The tests on what is left are
-// uniform first: a short row, one vector per lane or less, is bound by what it issues.
+// What is left, at most four vectors per thread, is loaded at once too, each into a chain of its
+// own, and the up to three elements behind the last vector join those of the first lanes.  Up to
+// 64 elements take 16 lanes with up to four each: an element that only joins at the top of the
+// tree would round once more at the full sum's size.
 template <int kOp, int kThreads, class Int>
 __device__ __forceinline__ float reduce_span(const float* x, Int len, int t) {
-  if (len <= kThreads) return t < len ? x[t] : identity<kOp>();
   constexpr int kUnroll = 4;
   float acc[4] = {identity<kOp>(), identity<kOp>(), identity<kOp>(), identity<kOp>()};
+  const auto total = [&] { return combine<kOp>(combine<kOp>(acc[0], acc[1]), combine<kOp>(acc[2], acc[3])); };
+  if (len <= 64) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (len > 16 * u && t < 16 && t + 16 * u < len) acc[u] = x[t + 16 * u];
+    return total();
+  }
   const auto add4 = [&](int u, f32x4_u v) {
     acc[u] = combine<kOp>(acc[u], combine<kOp>(combine<kOp>(v.x, v.y), combine<kOp>(v.z, v.w)));
   };
@@ -99,23 +105,22 @@ __device__ __forceinline__ float reduce_span(const float* x, Int len, int t) {
     for (int u = 0; u < kUnroll; ++u) add4(u, v[u]);
   }
   const int left = static_cast<int>(nvec - q0), rest = static_cast<int>(len - nvec * 4);
+  constexpr float kId = identity<kOp>();
+  const float tail = t < rest ? x[nvec * 4 + t] : kId;
   f32x4_u v[kUnroll];
-  float tail[3] = {identity<kOp>(), identity<kOp>(), identity<kOp>()};
 #pragma unroll
   for (int u = 0; u < kUnroll; ++u) {
-    v[u] = f32x4_u{identity<kOp>(), identity<kOp>(), identity<kOp>(), identity<kOp>()};
-    if (left > u * kThreads && t + u * kThreads < left) v[u] = load4(x + 4 * (q0 + t + u * kThreads));
-  }
-  if (rest > 0 && t == left % kThreads) {
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-      if (i < rest) tail[i] = x[nvec * 4 + i];
+    if (u > 0 && left <= u * kThreads) break;  // uniform
+    v[u] = f32x4_u{kId, kId, kId, kId};
+    if (t + u * kThreads < left) v[u] = load4(x + 4 * (q0 + t + u * kThreads));
   }
 #pragma unroll
-  for (int u = 0; u < kUnroll; ++u)
-    if (left > u * kThreads) add4(u, v[u]);
-  if (rest > 0) acc[3] = combine<kOp>(acc[3], combine<kOp>(combine<kOp>(tail[0], tail[1]), tail[2]));
-  return combine<kOp>(combine<kOp>(acc[0], acc[1]), combine<kOp>(acc[2], acc[3]));
+  for (int u = 0; u < kUnroll; ++u) {
+    if (u > 0 && left <= u * kThreads) break;
+    add4(u, v[u]);
+  }
+  acc[3] = combine<kOp>(acc[3], tail);
+  return total();
 }
 
 // Combines one value per thread of a kThreads-thread workgroup; every thread gets the result.

@@ -93,7 +93,8 @@ def test_split_reduction_on_a_side_stream_and_in_a_graph(device):
         assert torch.equal(out, want), k
 
 
-@pytest.mark.parametrize("rows,cols", [(512, 65536), (512, 3000), (300, 100003), (1024, 4096)])
+@pytest.mark.parametrize("rows,cols", [(512, 65536), (512, 3000), (300, 100003), (1024, 4096), (60000, 7),
+                                       (60000, 17), (60000, 33), (60000, 64), (60000, 67)])
 def test_row_sums_round_like_a_binary_tree(device, rows, cols):
     # the last additions of a sum carry its rounding error: in a binary tree their variances are
     # 1 + 1/2 + 1/4 + ... < 2 times that of one rounding, (2^-24)^2 / 3 relative at most.  A chain
