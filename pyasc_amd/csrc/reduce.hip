@@ -61,18 +61,22 @@ struct ReduceArgs {
   float* out;
   int64_t rows, cols;
   int64_t out_count;  // "all": number of output elements receiving the result
+  int64_t splits;     // dim 0, "all": workgroups that share one result's rows or elements
 };
 
 // First element of span i of n elements in `spans` parts, a multiple of 4.
 __device__ __forceinline__ int64_t span_start(int64_t n, int64_t i, int64_t spans) {
   const int64_t vecs = n / 4;
+  if (spans == 1) return i == 0 ? 0 : n;  // without the divisions, 0.4 us of a small launch
   return i == spans ? n : (vecs / spans * i + vecs % spans * i / spans) * 4;
 }
 
-// 16 bytes of fp32 at element alignment, streamed once.
+// 16 bytes of fp32 at element alignment; kStream: read once, not kept in the caches.
 typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+template <bool kStream = true>
 __device__ __forceinline__ f32x4_u load4(const float* p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const f32x4_u*>(p));
+  if constexpr (kStream) return __builtin_nontemporal_load(reinterpret_cast<const f32x4_u*>(p));
+  return *reinterpret_cast<const f32x4_u*>(p);
 }
 
 // Elements [0, len) of x by the kThreads threads of a group (t: the thread's index in it):
@@ -177,7 +181,7 @@ __global__ void __launch_bounds__(1024) reduce_cols_kernel(ReduceArgs p) {
   __shared__ float4 part[16][16];
   const int t = threadIdx.x, lane_c = t & 15;
   const int64_t c = static_cast<int64_t>(blockIdx.x) * kColsPerBlock + lane_c * 4;
-  const int64_t r0 = p.rows * blockIdx.y / gridDim.y, r1 = p.rows * (blockIdx.y + 1) / gridDim.y;
+  const int64_t r0 = p.rows * blockIdx.y / p.splits, r1 = p.rows * (blockIdx.y + 1) / p.splits;
   const int left = static_cast<int>(p.cols - c < 4 ? p.cols - c : 4);  // columns of this lane
   float acc[4] = {identity<kOp>(), identity<kOp>(), identity<kOp>(), identity<kOp>()};
   int64_t r = r0 + (t >> 4);
@@ -222,10 +226,15 @@ __global__ void __launch_bounds__(1024) reduce_cols_kernel(ReduceArgs p) {
   }
 }
 
-// dim 0 of few rows or very many columns: four columns per thread, eight rows' loads in flight.
-template <int kOp>
+// dim 0 of few rows or very many columns: four columns per thread, eight rows' loads in flight,
+// the last rows' at once too, one 16-byte store.  kStream only where x is larger than the L2s and
+// made of aligned vectors: a smaller x may be in the L2 from its producer, and two threads share
+// the lines of a misaligned row.  us, a thread per column before, here, x in the L2 / x from HBM:
+// 31x65537 4.5, 4.6 / 14.1, 6.0; 20x262144 3.7, 2.8 / 10.7, 5.9; 31x1000003 23.2, 24.5 / 36, 29;
+// 1x4194304 6.4, 4.9 / 11.3, 7.8; 24x4194304 (streamed) 107, 84 / 113, 84.
+template <int kOp, bool kStream>
 __global__ void __launch_bounds__(256) reduce_wide_cols_kernel(ReduceArgs p) {
-  const int64_t c = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
+  const int64_t c = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 4;
   if (c >= p.cols) return;
   float acc[4] = {identity<kOp>(), identity<kOp>(), identity<kOp>(), identity<kOp>()};
   const int left = static_cast<int>(p.cols - c < 4 ? p.cols - c : 4);
@@ -235,26 +244,32 @@ __global__ void __launch_bounds__(256) reduce_wide_cols_kernel(ReduceArgs p) {
 #pragma unroll
       for (int i = 0; i < 3; ++i)
         if (i < left) acc[i] = combine<kOp>(acc[i], x[r * p.cols + i]);
-  } else {
-    int64_t r = 0;
-    for (; r + 7 < p.rows; r += 8) {
-      f32x4_u v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = load4(x + (r + u) * p.cols);
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i] = combine<kOp>(acc[i], v[u][i]);
-    }
-    for (; r < p.rows; ++r) {
-      const f32x4_u v = load4(x + r * p.cols);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = combine<kOp>(acc[i], v[i]);
-    }
+    for (int i = 0; i < 3; ++i)
+      if (i < left) p.out[c + i] = acc[i];
+    return;
   }
+  const auto take = [&](f32x4_u v) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    if (i < left) p.out[c + i] = acc[i];
+    for (int i = 0; i < 4; ++i) acc[i] = combine<kOp>(acc[i], v[i]);
+  };
+  constexpr int kUnroll = 8;
+  int64_t r = 0;
+  f32x4_u v[kUnroll];
+  for (; r + kUnroll <= p.rows; r += kUnroll) {
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) v[u] = load4<kStream>(x + (r + u) * p.cols);
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) take(v[u]);
+  }
+  const int rest = static_cast<int>(p.rows - r);
+#pragma unroll
+  for (int u = 0; u < kUnroll - 1; ++u)
+    if (u < rest) v[u] = load4<kStream>(x + (r + u) * p.cols);
+#pragma unroll
+  for (int u = 0; u < kUnroll - 1; ++u)
+    if (u < rest) take(v[u]);
+  *reinterpret_cast<f32x4_u*>(p.out + c) = f32x4_u{acc[0], acc[1], acc[2], acc[3]};
 }
 
 // all elements: workgroup s reduces elements [s*n/grid, (s+1)*n/grid); the result is written to
@@ -262,9 +277,9 @@ __global__ void __launch_bounds__(256) reduce_wide_cols_kernel(ReduceArgs p) {
 template <int kOp>
 __global__ void __launch_bounds__(1024) reduce_all_kernel(ReduceArgs p) {
   const int64_t n = p.rows * p.cols;
-  const int64_t e0 = span_start(n, blockIdx.x, gridDim.x), e1 = span_start(n, blockIdx.x + 1, gridDim.x);
+  const int64_t e0 = span_start(n, blockIdx.x, p.splits), e1 = span_start(n, blockIdx.x + 1, p.splits);
   const float total = block_combine<kOp, 1024>(reduce_span<kOp, 1024>(p.x + e0, e1 - e0, threadIdx.x));
-  if (gridDim.x > 1) {
+  if (p.splits > 1) {
     if (threadIdx.x == 0) p.out[blockIdx.x] = total;
     return;
   }
@@ -293,18 +308,30 @@ int64_t reduce_splits(int64_t rows, int64_t cols, int dim) {
 }
 
 template <int kOp>
-void launch_cols(const ReduceArgs& p, int64_t splits, hipStream_t s) {
-  const dim3 grid(static_cast<uint32_t>(asc::ceil_div(p.cols, kColsPerBlock)), static_cast<uint32_t>(splits));
+void launch_cols(const ReduceArgs& p, hipStream_t s) {
+  const dim3 grid(static_cast<uint32_t>(asc::ceil_div(p.cols, kColsPerBlock)), static_cast<uint32_t>(p.splits));
   hipLaunchKernelGGL(reduce_cols_kernel<kOp>, grid, dim3(1024), 0, s, p);
 }
 
-// ws: room for the partial results of `splits` groups (null: splits is 1)
 template <int kOp>
-int32_t launch_reduce(const ReduceArgs& p, int dim, int64_t splits, float* ws, hipStream_t s) {
+void launch_wide_cols(const ReduceArgs& p, hipStream_t s) {
+  // a wave per workgroup spreads fewer than 2^18 columns over the CUs (31x65537: 4.6 us, 5.3 with
+  // four); past that four are the better (31x1000003: 27.7 us with one, 24.5)
+  const int threads = p.cols < (int64_t{1} << 18) ? 64 : 256;
+  const bool stream = asc::aligned16(p.x) && p.cols % 4 == 0 && p.rows * p.cols > (int64_t{8} << 20);
+  const auto kernel = stream ? reduce_wide_cols_kernel<kOp, true> : reduce_wide_cols_kernel<kOp, false>;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(asc::ceil_div(p.cols, 4 * threads))), dim3(threads), 0, s, p);
+}
+
+// ws: room for the partial results of p.splits groups (null: p.splits is 1)
+template <int kOp>
+int32_t launch_reduce(const ReduceArgs& p, int dim, float* ws, hipStream_t s) {
   if (dim == 1) {
-    // A wave per row keeps HBM busy from about 1024 rows up (16384x4096: 6.4 TB/s); fewer rows
-    // of 2048 columns or more take a workgroup each.  One dispatch covers fewer than 2^32 threads.
-    const bool wave_rows = p.rows >= 1024 || p.cols < 2048;
+    // A wave per row keeps HBM busy from about 1024 rows up (16384x4096: 6.0 TB/s).  Fewer rows of
+    // 2048 columns or more take a workgroup each while the rows are long for their number: us with a
+    // wave, a workgroup, x from HBM: 512x2048 3.1, 2.7; 768x4096 4.6, 4.5; 1023x2048 3.5, 4.1;
+    // 1023x8192 8.2, 7.7.  One dispatch covers fewer than 2^32 threads.
+    const bool wave_rows = p.rows >= 1024 || p.cols < 2048 || p.cols < 4 * p.rows;
     const int64_t blocks = wave_rows ? asc::ceil_div(p.rows, 4) : p.rows;
     ASC_REQUIRE(blocks * 256 < (int64_t{1} << 32), ASC_ERR_UNSUPPORTED, "asc_reduce_f32: %lld rows exceed one launch",
                 static_cast<long long>(p.rows));
@@ -315,20 +342,20 @@ int32_t launch_reduce(const ReduceArgs& p, int dim, int64_t splits, float* ws, h
     }
   } else if (dim == 0) {
     if (wide_cols(p.rows, p.cols)) {
-      hipLaunchKernelGGL(reduce_wide_cols_kernel<kOp>, dim3(static_cast<uint32_t>(asc::ceil_div(p.cols, 1024))),
-                         dim3(256), 0, s, p);
-    } else if (splits == 1) {
-      launch_cols<kOp>(p, 1, s);
+      launch_wide_cols<kOp>(p, s);
+    } else if (p.splits == 1) {
+      launch_cols<kOp>(p, s);
     } else {
-      launch_cols<kOp>(ReduceArgs{p.x, ws, p.rows, p.cols, 0}, splits, s);
-      launch_cols<kOp>(ReduceArgs{ws, p.out, splits, p.cols, 0}, 1, s);
+      launch_cols<kOp>(ReduceArgs{p.x, ws, p.rows, p.cols, 0, p.splits}, s);
+      launch_cols<kOp>(ReduceArgs{ws, p.out, p.splits, p.cols, 0, 1}, s);
     }
-  } else if (splits == 1) {
+  } else if (p.splits == 1) {
     hipLaunchKernelGGL(reduce_all_kernel<kOp>, dim3(1), dim3(1024), 0, s, p);
   } else {
-    hipLaunchKernelGGL(reduce_all_kernel<kOp>, dim3(static_cast<uint32_t>(splits)), dim3(1024), 0, s,
-                       ReduceArgs{p.x, ws, p.rows, p.cols, 0});
-    hipLaunchKernelGGL(reduce_all_kernel<kOp>, dim3(1), dim3(1024), 0, s, ReduceArgs{ws, p.out, 1, splits, p.out_count});
+    hipLaunchKernelGGL(reduce_all_kernel<kOp>, dim3(static_cast<uint32_t>(p.splits)), dim3(1024), 0, s,
+                       ReduceArgs{p.x, ws, p.rows, p.cols, 0, p.splits});
+    hipLaunchKernelGGL(reduce_all_kernel<kOp>, dim3(1), dim3(1024), 0, s,
+                       ReduceArgs{ws, p.out, 1, p.splits, p.out_count, 1});
   }
   return asc::check_launch("asc_reduce_f32");
 }
@@ -533,10 +560,9 @@ extern "C" int32_t asc_reduce_f32_ws(int32_t op, const float* x, float* out, int
   if (results == 0) return ASC_OK;
   ASC_REQUIRE(rows > 0 && cols > 0, ASC_ERR_INVALID_ARG, "asc_reduce_f32: empty input");
   ASC_REQUIRE(x && out, ASC_ERR_INVALID_ARG, "asc_reduce_f32: null buffer");
-  const ReduceArgs p{x, out, rows, cols, out_count};
-  int64_t splits = 1;
+  ReduceArgs p{x, out, rows, cols, out_count, 1};
   if (workspace != nullptr) {
-    splits = reduce_splits(rows, cols, dim);
+    p.splits = reduce_splits(rows, cols, dim);
     const int64_t need = asc_reduce_f32_workspace(rows, cols, dim);
     ASC_REQUIRE(workspace_bytes >= need, ASC_ERR_INVALID_ARG,
                 "asc_reduce_f32_ws: the partial results need %lld bytes, the workspace holds %lld", (long long)need,
@@ -547,10 +573,10 @@ extern "C" int32_t asc_reduce_f32_ws(int32_t op, const float* x, float* out, int
   float* ws = static_cast<float*>(workspace);
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (op) {
-    case kSum: return launch_reduce<kSum>(p, dim, splits, ws, s);
-    case kMax: return launch_reduce<kMax>(p, dim, splits, ws, s);
-    case kMin: return launch_reduce<kMin>(p, dim, splits, ws, s);
-    default: return launch_reduce<kProd>(p, dim, splits, ws, s);
+    case kSum: return launch_reduce<kSum>(p, dim, ws, s);
+    case kMax: return launch_reduce<kMax>(p, dim, ws, s);
+    case kMin: return launch_reduce<kMin>(p, dim, ws, s);
+    default: return launch_reduce<kProd>(p, dim, ws, s);
   }
 }
 

@@ -105,3 +105,23 @@ def test_row_sums_round_like_a_binary_tree(device, rows, cols):
     ref = x.double().sum(1)
     rms = ((out.double() - ref) / ref).square().mean().sqrt().item()
     assert rms <= 2.0 ** -24 * (2 / 3) ** 0.5, rms
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("rows,cols", [(1, 262143), (2, 262144), (7, 65537), (8, 65536), (9, 262147), (15, 1001),
+                                       (31, 270604), (16, 524292), (17, 524292), (33, 262145), (512, 4096), (512, 4095),
+                                       (255, 2048), (257, 2048), (1023, 8184)])
+def test_few_rows_and_row_lines(device, rows, cols, offset):
+    # columns over one or four waves per workgroup, x above and below the size that is streamed,
+    # 16-byte aligned or not, 1..7 rows behind a step of eight, and rows on both sides of the line
+    # between a wave and a workgroup per row
+    g = torch.Generator(device=device).manual_seed(rows + cols)
+    x = torch.rand(rows * cols + offset, generator=g, device=device)[offset:].view(rows, cols)
+    for dim, n in ((0, cols), (1, rows)):
+        out = torch.full((n + 8,), -7.0, device=device)
+        kernels.reduce_f32(x, out[4:n + 4], "sum", dim)
+        ref = x.double().sum(dim)
+        assert ((out[4:n + 4].double() - ref).abs() <= x.shape[dim] * 2.0 ** -24 * ref).all()
+        kernels.reduce_f32(x, out[4:n + 4], "max", dim)
+        assert torch.equal(out[4:n + 4], x.amax(dim))
+        assert (out[:4] == -7.0).all() and (out[n + 4:] == -7.0).all()
