@@ -335,7 +335,7 @@ __device__ __forceinline__ void two_pass_body(const void* x, void* out, int64_t 
   const int t = threadIdx.x;
   const int64_t r = blockIdx.x;
   const float* row = p.x + r * p.stride;
-  const int nvec = (p.len + 3) / 4;
+  const int nvec = p.len / 4 + (p.len % 4 != 0);
   OnlineSum acc;
   float mn = INFINITY;
   constexpr int kChunk = 8;
@@ -349,7 +349,11 @@ __device__ __forceinline__ void two_pass_body(const void* x, void* out, int64_t 
       }
     } else {
 #pragma unroll
-      for (int u = 0; u < kChunk; ++u) v[u] = load_vec(row, q + kThreads * u, p.len, kPad);
+      for (int u = 0; u < kChunk; ++u) {
+        // a vector past the row is not asked for: its first element may not fit an int
+        v[u] = make_float4(kPad, kPad, kPad, kPad);
+        if (q + kThreads * u < nvec) v[u] = load_vec(row, q + kThreads * u, p.len, kPad);
+      }
     }
     float m = -INFINITY;
 #pragma unroll
@@ -453,16 +457,18 @@ struct HalfRow {
                                      int32_t len) {
     const uint16_t* row = xs + r * stride;
     h = static_cast<int>(reinterpret_cast<uintptr_t>(row) & 15) >> 1;
-    const bool inside = (h == 0 || r * stride >= 8) && (((h + len) & 7) == 0 || (rows - 1 - r) * stride >= 8);
-    // Where an aligned vector would leave the tensor (its first or last row), vectors start at
-    // the row, and the last one is moved back over elements that the one before it holds.
+    const bool inside = (h == 0 || r * stride >= 8) && (((h + (len & 7)) & 7) == 0 || (rows - 1 - r) * stride >= 8) &&
+                        len <= INT32_MAX - 16;
+    // Where an aligned vector would leave the tensor (its first or last row), or its end an int,
+    // vectors start at the row, and the last one is moved back over elements that the one before
+    // it holds.
     if (!inside) h = 0;
     x = row - h;
     out = outs + r * stride - h;
     end = h + len;
     last = inside ? end : len - 8;
   }
-  __device__ __forceinline__ int vectors() const { return (end + 7) / 8; }
+  __device__ __forceinline__ int vectors() const { return end / 8 + (end % 8 != 0); }
   __device__ __forceinline__ bool tiny() const { return last < 0; }  // less than a vector to read
   __device__ __forceinline__ int first(int q) const { return min(8 * q, last); }
 

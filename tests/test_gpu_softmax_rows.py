@@ -3,6 +3,8 @@ or two passes), with remainders of a vector, rows that start on any element, par
 and fused blocks, and rows with infinities and NaN, against the fp64 softmax.  fp32: x - max is
 rounded to fp32 (as the reference does), which alone moves exp by |x - max| * 2^-24 of its
 value; exp, the sum, the reciprocal and the product add at most 8 ulp.  fp16: one ulp."""
+import math
+
 import pytest
 import torch
 
@@ -97,3 +99,20 @@ def test_infinities_and_nan(device, dtype, cols):
     assert torch.equal(torch.isnan(out), torch.isnan(ref))
     for r in (0, 4, 5, 6):
         _check(out[r:r + 1], x[r:r + 1], dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("short", [0, 3, 9, 20000])
+def test_longest_rows(device, dtype, short):
+    # rows whose vectors and chunks end at or past 2^31 elements, starting on an odd element: all of
+    # the sum comes from the two ends, the rest is 0, and nothing around the row changes
+    cols = 2 ** 31 - 1 - short
+    x = torch.full((cols + 1,), -200.0, dtype=dtype, device=device)[1:]
+    x[0], x[-1] = 11.0, 10.0
+    buf = torch.full((cols + 2,), 7.0, dtype=dtype, device=device)
+    out = buf[1:-1]
+    kernels.softmax_rows(x, out, 1, cols, cols, 16)
+    torch.cuda.synchronize()
+    for at, want in ((0, 1 / (1 + math.exp(-1.0))), (-1, 1 / (1 + math.exp(1.0)))):
+        assert abs(out[at].item() - want) <= want * (2.0 ** -10 if dtype == torch.float16 else 17 * 2.0 ** -24), at
+    assert (out[1:-1] == 0).all() and buf[0] == 7.0 and buf[-1] == 7.0
