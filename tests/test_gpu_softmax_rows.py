@@ -55,6 +55,20 @@ def _row_lengths(device, dtype, cols, offset, rows):
     assert (buf[:offset] == 7.0).all() and (buf[offset + rows * cols:] == 7.0).all()
 
 
+@pytest.mark.parametrize("cols", [64, 100, 192, 200, 256, 384, 400, 512])
+def test_short_rows_round_their_sum_once(device, cols):
+    # Rows of nearly equal values: what a row's results have in common is the rounding of the sum
+    # and of its reciprocal.  One rounding each has variances 1 / m^2 + m^2 / 4 <= 1.25 for a sum of
+    # mantissa m, in units of (2^-24)^2 / 3; chains of up to 8 additions in 16 lanes add at most
+    # 16 * (1 + 4 + ... + 64) / 64 / 256.  A tree that rounds at every level has 1/2 + 1/4 + 1/8 more.
+    x = torch.randn((8192, cols), generator=torch.Generator(device=device).manual_seed(cols), device=device) * 0.1
+    out = torch.empty_like(x)
+    kernels.softmax_rows(x, out, 8192, cols, cols, 16)
+    ref = torch.softmax(x.double(), dim=1)
+    scale = (out.double() / ref).mean(dim=1) - 1  # what a row's results have in common
+    assert scale.square().mean().sqrt().item() <= 2.0 ** -24 * ((1.25 + 16 * 204 / 64 / 256) / 3) ** 0.5
+
+
 @pytest.mark.parametrize("dtype,cols,tile", [(torch.float32, 20000, 17001), (torch.float16, 20000, 17001),
                                              (torch.float16, 300, 77), (torch.float32, 300, 77)])
 def test_partial_tiles_and_fused_blocks(device, dtype, cols, tile):
