@@ -164,7 +164,7 @@ void dispatch(Plan& p) {
     p.kernel = kWideF16;
     p.block = 1024;
   } else if (p.kernel == kF16) {
-    const int64_t groups = asc::ceil_div(p.rows, asc::softmax::f16_rows_per_block(p.len, p.rows));
+    const int64_t groups = asc::ceil_div(p.rows, asc::softmax::f16_rows_per_block(p.len, p.rows, p.flag != 0));
     if (groups < p.grid) p.grid = groups;
   }
 }

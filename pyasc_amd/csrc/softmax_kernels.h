@@ -11,9 +11,10 @@
 //
 // Every body takes the same six arguments,
 //   (x, out, rows, stride, len, flag)
-// where flag is "rows start 16-byte aligned" for the register-resident and f16
-// bodies (which load and store at element alignment and do not need it) and the
-// pad count (tile - num_cols) for the padded bodies.
+// where flag is "rows start 16-byte aligned" for the fp32 bodies (which load and
+// store at element alignment and do not need it), "rows are made of aligned
+// 16-byte vectors" for the f16 bodies and the pad count (tile - num_cols) for the
+// padded bodies.
 //
 // HBM-bound (one read + one write of every element).  Rows up to 49152 fp32 or 65529
 // fp16 columns stay in registers: 16 lanes, a wave or a workgroup per row, by its
@@ -586,6 +587,38 @@ __device__ __forceinline__ void f16_rows(const uint16_t* x, uint16_t* out, int64
   }
 }
 
+// Few rows that are not made of aligned vectors, element by element: kPer per lane, a row per
+// group of kLanes of the workgroup's threads.  With few rows the latency of one counts, and the
+// masks of a vector at a row's ends cost more of it than loads of an element each (an element per
+// thread before, vectors, here; us): 16x122 2.3, 2.7, 2.0; 128x506 2.9, 3.3, 2.2; 512x1017 3.8,
+// 3.8, 2.6; 1000x122 2.9, 2.9, 2.1; 1000x1017 4.7, 4.0, 3.0.
+template <int kPer, int kLanes>
+__device__ __forceinline__ void f16_element_rows(const uint16_t* x, uint16_t* out, int64_t rows, int64_t stride,
+                                                 int32_t len, float (*red)[16]) {
+  constexpr int kGroups = 256 / kLanes;
+  const int t = threadIdx.x % kLanes;
+  for (int64_t r = static_cast<int64_t>(blockIdx.x) * kGroups + threadIdx.x / kLanes; r < rows;
+       r += static_cast<int64_t>(gridDim.x) * kGroups) {
+    float f[kPer];
+    float m = -INFINITY, s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      f[j] = t + kLanes * j < len ? half_at(x + r * stride, t + kLanes * j) : -INFINITY;
+      m = fmaxf(m, f[j]);
+    }
+    m = group_max<kLanes>(m, red[0]);
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      f[j] = exp_flush(f[j] - m);
+      s += f[j];
+    }
+    const float rs = 1.0f / group_sum<kLanes>(s, red[1]);
+#pragma unroll
+    for (int j = 0; j < kPer; ++j)
+      if (t + kLanes * j < len) out[r * stride + t + kLanes * j] = to_half(f[j] * rs);
+  }
+}
+
 // Longer rows, one per workgroup, in two passes.
 template <int kThreads>
 __device__ __forceinline__ void f16_long_rows(const uint16_t* x, uint16_t* out, int64_t rows, int64_t stride,
@@ -624,16 +657,29 @@ __device__ __forceinline__ void f16_long_rows(const uint16_t* x, uint16_t* out, 
 // row's own latency counts and more lanes are better (300x333: 3.2 us with a wave, 4.1 with 16
 // lanes, even at about 2000 rows; 1000x4000: 5.7 with a workgroup, 8x4000: 3.1, 4.7 with a wave,
 // even at about 1000 rows).
-constexpr int32_t f16_rows_per_block(int32_t len, int64_t rows) {
+constexpr bool f16_by_elements(int32_t len, int64_t rows, bool aligned) {
+  return !aligned && len <= 1017 && rows <= 1024;
+}
+constexpr int32_t f16_rows_per_block(int32_t len, int64_t rows, bool aligned) {
+  if (f16_by_elements(len, rows, aligned)) return len <= 256 ? 4 : 1;
   if (len <= 505) return len <= 121 || rows > 2048 ? 16 : 4;
   return len <= 1017 || (len <= 4089 && rows > 1024) ? 4 : 1;
 }
 
+// aligned: rows are made of 16-byte vectors at aligned addresses.
 __device__ __forceinline__ void f16_body(const void* xv, void* outv, int64_t rows, int64_t stride, int32_t len,
-                                         int32_t) {
+                                         int32_t aligned) {
   __shared__ float red[2][16];
   const uint16_t* x = static_cast<const uint16_t*>(xv);
   uint16_t* out = static_cast<uint16_t*>(outv);
+  if (f16_by_elements(len, rows, aligned != 0)) {
+    if (len <= 64) return f16_element_rows<1, 64>(x, out, rows, stride, len, red);
+    if (len <= 128) return f16_element_rows<2, 64>(x, out, rows, stride, len, red);
+    if (len <= 256) return f16_element_rows<4, 64>(x, out, rows, stride, len, red);
+    if (len <= 512) return f16_element_rows<2, 256>(x, out, rows, stride, len, red);
+    if (len <= 768) return f16_element_rows<3, 256>(x, out, rows, stride, len, red);
+    return f16_element_rows<4, 256>(x, out, rows, stride, len, red);
+  }
   if (len <= 121) return f16_rows<1, 16, 256>(x, out, rows, stride, len, red);
   if (len <= 505 && rows <= 2048) return f16_rows<1, 64, 256>(x, out, rows, stride, len, red);
   if (len > 1017 && rows <= 1024) {
@@ -656,7 +702,7 @@ __device__ __forceinline__ void f16_body(const void* xv, void* outv, int64_t row
   f16_long_rows<256>(x, out, rows, stride, len, red);
 }
 
-// 1024 threads per row: few rows, and rows past 16377 columns (registers up to 65529).
+// 1024 threads per row, for rows past 16377 columns (registers up to 65529).
 __device__ __forceinline__ void f16_wide_body(const void* xv, void* outv, int64_t rows, int64_t stride, int32_t len,
                                               int32_t) {
   __shared__ float red[2][16];

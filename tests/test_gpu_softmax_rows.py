@@ -55,6 +55,14 @@ def _row_lengths(device, dtype, cols, offset, rows):
     assert (buf[:offset] == 7.0).all() and (buf[offset + rows * cols:] == 7.0).all()
 
 
+@pytest.mark.parametrize("rows", [1, 3, 1024, 1025])
+@pytest.mark.parametrize("cols", [1, 63, 64, 65, 127, 128, 129, 255, 257, 511, 512, 513, 767, 769, 1016, 1017, 1018])
+def test_few_half_rows(device, cols, rows):
+    # rows taken by elements or by vectors, by their number, length and alignment
+    for offset in (0, 1, 4):
+        _row_lengths(device, torch.float16, cols, offset, rows)
+
+
 @pytest.mark.parametrize("cols", [64, 100, 192, 200, 256, 384, 400, 512])
 def test_short_rows_round_their_sum_once(device, cols):
     # Rows of nearly equal values: what a row's results have in common is the rounding of the sum
