@@ -122,8 +122,8 @@ const TileFn kTileF32[asc::tile::kNumF32] = ASC_TILE_TABLE_F32(asc_tile_f32_);
 
 // The tile launch that takes the call of a checked, non-empty MmLaunch, or T.index < 0 when
 // L's own kernel runs it: K == 0 (no operand may be read), the tile-aligned loop on its own
-// 256x256 tiles (4096^3 bf16: 114.8 us against 115.8), and fp32 of up to 256 16x16 blocks on
-// operands that are not 16-byte aligned (100x301x501: 6.6 us against 7.6).
+// 256x256 tiles (4096^3 bf16: 114.8 us against 115.8), and fp32 in 16x16 blocks: up to 256 of them on
+// operands that are not 16-byte aligned (100x301x501: 6.6 us against 7.6), and short products.
 void make_tile(int32_t in_dtype, int32_t out_dtype, const MmLaunch& L, TileLaunch& T) {
   T = TileLaunch{};
   const GemmArgs& g = L.p;
@@ -133,6 +133,8 @@ void make_tile(int32_t in_dtype, int32_t out_dtype, const MmLaunch& L, TileLaunc
   if (in_dtype == ASC_DT_FLOAT32) {
     if (!dma && ((g.M + 15) / 16) * static_cast<int64_t>((g.N + 15) / 16) <= asc::tile::kCus) return;
     asc::tile::choose_f32(dma, g.M, g.N, g.K, T);
+    const bool blocks = L.kernel % kKinds == 4;
+    if (blocks && T.index >= 0 && asc::tile::f32_prefers_blocks(T.index, T.us, g.M, g.N, g.K)) T.index = -1;
   } else {
     asc::tile::choose_mfma(es, dma, g.M, g.N, g.K, T);
     if (T.index == asc::tile::kD256x256 && (L.kernel % kKinds & 1) == 0) T.index = -1;

@@ -261,7 +261,8 @@ __device__ __forceinline__ void gemm_f32_mfma_body(const GemmArgs& p) {
   const bool a_ok = m0 + r < M, b_ok = n0 + r < N;
   const float* arow = a + static_cast<int64_t>(a_ok ? m0 + r : 0) * lda;
   const float* bcol = b + (b_ok ? n0 + r : 0);
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  // one chain per MFMA of a group, summed in pairs: half the rounding of one chain
+  f32x4 acc[4] = {};
   const int groups = (K + 15) / 16;
   for (int g = wave; g < groups; g += 4) {
     const int kb = 16 * g + 4 * q;
@@ -274,14 +275,12 @@ __device__ __forceinline__ void gemm_f32_mfma_body(const GemmArgs& p) {
       bv[j] = b_ok && k_ok ? bcol[static_cast<int64_t>(k) * ldb] : 0.f;
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j], bv[j], acc, 0, 0, 0);
+    for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j], bv[j], acc[j], 0, 0, 0);
   }
-  partial[wave][lane] = acc;
+  partial[wave][lane] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
   __syncthreads();
   if (wave != 0) return;
-  acc = partial[0][lane];
-#pragma unroll
-  for (int w = 1; w < 4; ++w) acc += partial[w][lane];
+  const f32x4 sum = (partial[0][lane] + partial[1][lane]) + (partial[2][lane] + partial[3][lane]);
   const int n = n0 + r;
   if (n >= N) return;
   const float bias_n = epi.bias_at(n);
@@ -289,7 +288,7 @@ __device__ __forceinline__ void gemm_f32_mfma_body(const GemmArgs& p) {
   for (int rr = 0; rr < 4; ++rr) {
     const int m = m0 + 4 * q + rr;
     if (m >= M) continue;
-    const float v = epi(acc[rr], bias_n);
+    const float v = epi(sum[rr], bias_n);
     const int64_t off = static_cast<int64_t>(m) * ldc + n;
     if constexpr (kOut == kOutF32) static_cast<float*>(c)[off] = v;
     else if constexpr (kOut == kOutF16) static_cast<uint16_t*>(c)[off] = asc::f32_to_f16_rne(v);

@@ -129,6 +129,31 @@ constexpr Variant kF32[kNumF32] = {{"128x128", 128, 128, 512, 0.97f, 4.0f},    {
 
 constexpr int kCus = 256;
 
+// A launch of the 16x16-block kernel of matmul_kernels.h, in the units of the variants' models: a
+// short start, then a chain of loads along K (with few rows most of A's are masked) or, with many
+// blocks, the rate at which they get through K.  Against it the tiles' models, which rank tiles on
+// products of some length, leave out part of their start.  The lines end where the tiles' time per
+// k-tile is the smaller one throughout.  Measured us, blocks and tiles: 64x64x16 2.7, 3.4; 256x256x64
+// 3.0, 3.5; 512x512x32 3.5, 3.7; 16x4096x128 3.7, 3.8; 1x64x256 3.3, 4.0; 256x256x256 4.9, 4.3;
+// unaligned 260x260x57 2.9, 4.9; 300x301x100 3.6, 5.1; 113x1390x137 5.0, 6.0; 512x257x192 6.7, 5.7.
+inline double f32_blocks_us(bool aligned, int64_t M, int64_t N, int64_t K) {
+  const double blocks = static_cast<double>((M + 15) / 16) * static_cast<double>((N + 15) / 16);
+  const double chain = M <= 8 ? 0.0052 : 0.011, rate = (aligned ? 3.4e-5 : 4.2e-5) * blocks;
+  const double along_k = static_cast<double>(K) * (chain > rate ? chain : rate), starts = 0.0008 * blocks;
+  return 0.8 + (along_k > starts ? along_k : starts);
+}
+inline bool f32_prefers_blocks(int index, double us, int64_t M, int64_t N, int64_t K) {
+  constexpr double kStart[kNumF32] = {0.0, 0.4, 0.0, 0.0, 1.2, 1.8}, kLeast[kNumF32] = {0.0, 3.5, 2.3, 0.0, 0.0, 0.0};
+  const bool aligned = index < kFA128x128;
+  if (K > (M <= 8 ? 512 : aligned ? 160 : 320)) return false;
+  const Variant& v = kF32[index];
+  const int64_t tiles = ((M + v.bm - 1) / v.bm) * ((N + v.bn - 1) / v.bn);
+  const double rounds = static_cast<double>((tiles + kCus - 1) / kCus);
+  us += rounds * kStart[index];
+  if (us < rounds * kLeast[index]) us = rounds * kLeast[index];
+  return f32_blocks_us(aligned, M, N, K) <= us;
+}
+
 // One tile launch: the variant's index in its type's kernel table, name, arguments, grid.
 struct TileLaunch {
   int index = -1;  // -1: no variant takes the call
@@ -136,6 +161,7 @@ struct TileLaunch {
   TileArgs p{};
   int64_t blocks = 0;
   int threads = 0;
+  double us = 0.0;  // modelled time
 };
 
 // Picks among variants [first, last) of `table` the one with the least modelled time whose
@@ -144,14 +170,13 @@ template <class Takes>
 inline void choose(const Variant* table, int first, int last, int64_t M, int64_t N, int64_t k_bytes, TileLaunch& L,
                    Takes takes) {
   const double ktiles = static_cast<double>(k_bytes) / 64.0;
-  double best = 0.0;
   for (int i = first; i < last; ++i) {
     const Variant& v = table[i];
     const int64_t tm = (M + v.bm - 1) / v.bm, tn = (N + v.bn - 1) / v.bn, tiles = tm * tn;
     if (tiles * v.threads >= (int64_t{1} << 32) || tiles >= (int64_t{1} << 31) || !takes(i)) continue;
     const double us = static_cast<double>((tiles + kCus - 1) / kCus) * (ktiles * v.per_ktile_us + v.fixed_us);
-    if (L.index >= 0 && us >= best) continue;
-    best = us;
+    if (L.index >= 0 && us >= L.us) continue;
+    L.us = us;
     L.index = i;
     L.name = v.name;
     L.blocks = tiles;

@@ -19,7 +19,7 @@ ALIGNED = [(1, 64, 64), (33, 40, 8), (31, 520, 1032), (17, 8200, 136), (65, 2056
            (1999, 4096, 72), (150, 4096, 4096), (1025, 2056, 136), (3001, 3008, 200), (2049, 4104, 4104)]
 # nothing aligned
 ODD = [(1, 1, 1), (3, 5, 7), (33, 31, 33), (64, 65, 1001), (127, 129, 63), (200, 301, 35), (200, 1001, 35), (257, 1001, 65),
-       (1001, 2003, 131), (3001, 2999, 97)]
+       (1001, 2003, 131), (3001, 2999, 97), (260, 261, 401)]
 SEEN = set()
 
 
@@ -120,3 +120,21 @@ def test_int8_tiles_are_exact(device, shape):
 def test_every_tile_kernel_ran(device):
     from pyasc_amd.launchers import MATMUL_CO_FUNCTIONS, MATMUL_I8_CO_FUNCTIONS
     assert {n for n in MATMUL_CO_FUNCTIONS + MATMUL_I8_CO_FUNCTIONS if "_tile_" in n} <= SEEN
+
+
+@pytest.mark.parametrize("shape", [(1, 64, 4), (8, 1024, 512), (16, 16, 16), (64, 64, 64), (100, 100, 128), (256, 256, 64),
+                                   (512, 512, 16), (260, 261, 57), (300, 257, 256), (9, 11007, 101)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_short_f32_products_take_blocks(device, shape):
+    # 16x16 blocks where a tile's start takes longer than the product
+    M, N, K = shape
+    g = torch.Generator(device=device).manual_seed(M + N + K)
+    a = torch.randn((M, K), generator=g, device=device)
+    b = torch.randn((K, N), generator=g, device=device)
+    bias = torch.randn(N, generator=g, device=device)
+    c = torch.full((M, N), 7.0, device=device)
+    kw = dict(bias=bias, leaky_alpha=0.25)
+    assert kernels.matmul_dispatch(a, b, c, **kw).kernel.decode() == "asc2_mm_f32_mfma_f32"
+    kernels.matmul(a, b, c, **kw)
+    torch.cuda.synchronize()
+    _check(c, a, b, bias, "leaky", 0.25)

@@ -118,3 +118,20 @@ def test_every_tile_kernel_is_reached():
         assert lib().asc_matmul_i8_dispatch(A, B, BIAS, C, M, N, K, 1, 0, ctypes.byref(p)) == 0
         seen.add(p.kernel.decode())
     assert {n for n in MATMUL_CO_FUNCTIONS + MATMUL_I8_CO_FUNCTIONS if "_tile_" in n} <= seen
+
+
+def test_short_f32_products_take_blocks():
+    # on both sides of each line: K, the number of blocks, the alignment, a few rows
+    def name(M, N, K, a=A):
+        rc, p = mm("asc_matmul_dispatch", F32, F32, M, N, K, K, N, N, a=a)
+        assert rc == 0
+        return p.kernel.decode()
+
+    blocks = "asc2_mm_f32_mfma_f32"
+    for M, N, K in ((1, 64, 4), (16, 16, 16), (64, 64, 64), (256, 256, 64), (512, 512, 16), (1, 4096, 256),
+                    (260, 261, 57), (113, 1390, 137), (1, 11007, 101), (300, 301, 100)):
+        assert name(M, N, K) == blocks, (M, N, K)
+    for M, N, K in ((64, 64, 256), (256, 256, 256), (1, 4096, 1024), (1024, 1024, 64), (2048, 2048, 16),
+                    (260, 261, 321), (1001, 1003, 101), (2049, 2049, 3)):
+        assert name(M, N, K) != blocks, (M, N, K)
+    assert name(64, 64, 256, a=A + 4) == blocks  # unaligned, up to 256 blocks: whatever K
