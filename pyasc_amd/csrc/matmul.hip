@@ -136,8 +136,9 @@ void make_tile(int32_t in_dtype, int32_t out_dtype, const MmLaunch& L, TileLaunc
     const bool blocks = L.kernel % kKinds == 4;
     if (blocks && T.index >= 0 && asc::tile::f32_prefers_blocks(T.index, T.us, g.M, g.N, g.K)) T.index = -1;
   } else {
-    asc::tile::choose_mfma(es, dma, g.M, g.N, g.K, T);
-    if (T.index == asc::tile::kD256x256 && (L.kernel % kKinds & 1) == 0) T.index = -1;
+    const bool fast = (L.kernel % kKinds & 1) == 0;
+    asc::tile::choose_mfma(es, dma, fast, g.M, g.N, g.K, T);
+    if (T.index == asc::tile::kD256x256 && fast) T.index = -1;
   }
   asc::gemm::TileArgs& p = T.p;
   p.a = g.a;

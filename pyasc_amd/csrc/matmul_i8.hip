@@ -74,8 +74,9 @@ void make_tile(int mode, const I8Launch& L, TileLaunch& T) {
   const I8Args& g = L.p;
   if (g.K == 0) return;
   const bool dma = asc::tile::dma_takes(g.a, g.b, g.N, g.K, g.K, g.N, 1);
-  asc::tile::choose_mfma(1, dma, g.M, g.N, g.K, T);
-  if (T.index == asc::tile::kD256x256 && L.kernel < 2) T.index = -1;
+  const bool fast = L.kernel < 2;
+  asc::tile::choose_mfma(1, dma, fast, g.M, g.N, g.K, T);
+  if (T.index == asc::tile::kD256x256 && fast) T.index = -1;
   asc::gemm::TileArgs& p = T.p;
   p.a = g.a;
   p.b = g.b;

@@ -195,13 +195,26 @@ inline bool dma_takes(const void* a, const void* b, int64_t N, int64_t K, int64_
          128 * ldb * es < kLimit;
 }
 
-// Fills the arguments and picks the variant for an fp16 / bf16 / int8 product (element size
-// `es`); 64x64k2 splits K over two groups, which only helps while a CU holds one tile.
-inline void choose_mfma(int es, bool dma, int64_t M, int64_t N, int64_t K, TileLaunch& L) {
+// Picks the variant for an fp16 / bf16 / int8 product (element size `es`); 64x64k2 splits K over
+// two groups, which only helps while a CU holds one tile.  aligned256: the tile-aligned loop of
+// gemm_direct.h takes the product (variant 256x256 stands for it).  From 129 of its tiles up, the
+// larger tiles are better than the model says where a round leaves CUs idle, as the others share more
+// of the L2 and of the power.  Up to 256 of its tiles that loop takes the product, above 192x128
+// has to be 15% better by the model (us, the better of the loop and 128x256, and 192x128: bf16
+// 3072x3072x4096 81, 93; 3072x4096x11008 232, 262; 6144x4096x11008 469, 518; 6144x6144x11008 783, 842;
+// int8 3072x3072x11008 110, 127; but 4608x4096x4096 180, 157).
+inline void choose_mfma(int es, bool dma, bool aligned256, int64_t M, int64_t N, int64_t K, TileLaunch& L) {
   if (dma) {
-    const int64_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
-    choose(kDma, 0, kNumDma, M, N, K * es, L,
-           [&](int i) { return i == kD64x64 ? tiles64 > kCus : i == kD64x64k2 ? tiles64 <= kCus : true; });
+    const int64_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64), tiles256 = ((M + 255) / 256) * ((N + 255) / 256);
+    const bool many = aligned256 && tiles256 > kCus / 2, one_round = many && tiles256 <= kCus;
+    choose(kDma, 0, one_round ? kD256x256 + 1 : kNumDma, M, N, K * es, L, [&](int i) {
+      return i == kD64x64 ? tiles64 > kCus : i == kD64x64k2 ? tiles64 <= kCus : !(many && i == kD192x128);
+    });
+    if (many && !one_round) {
+      TileLaunch other;
+      choose(kDma, kD192x128, kD192x128 + 1, M, N, K * es, other, [](int) { return true; });
+      if (other.index >= 0 && L.index >= 0 && other.us < 0.85 * L.us) L = other;
+    }
     return;
   }
   choose(kAny, 0, kNumAny, M, N, K * es, L, [](int) { return true; });

@@ -135,3 +135,24 @@ def test_short_f32_products_take_blocks():
                     (260, 261, 321), (1001, 1003, 101), (2049, 2049, 3)):
         assert name(M, N, K) != blocks, (M, N, K)
     assert name(64, 64, 256, a=A + 4) == blocks  # unaligned, up to 256 blocks: whatever K
+
+
+def test_tile_aligned_products_keep_their_loop():
+    # from 129 to 256 tiles of 256x256 every other tile is the slower one; above, 192x128 is where it
+    # fills about as many rounds
+    def names(M, N, K):
+        rc, p = mm("asc_matmul_dispatch", BF16, BF16, M, N, K, K, N, N)
+        q = _native.LaunchPlan()
+        assert rc == 0 and lib().asc_matmul_i8_dispatch(A, B, BIAS, C, M, N, K, 1, 0, ctypes.byref(q)) == 0
+        return p.kernel.decode(), q.kernel.decode()
+
+    for tm in range(1, 40):
+        for tn in (1, 3, 8, 12, 16, 24, 43):
+            for K in (64, 1024, 4096, 11008, 1 << 16):
+                if 128 < tm * tn <= 256:
+                    assert all("_fast_" in n for n in names(256 * tm, 256 * tn, K)), (tm, tn, K)
+    for M, N, K in ((6144, 4096, 11008), (5632, 4096, 11008), (6144, 6144, 4096), (2048, 11008, 11008)):
+        assert not any("192x128" in n for n in names(M, N, K)), (M, N, K)
+    assert all("192x128" in n for n in names(1536, 4096, 4096))  # one round of 192x128
+    assert all("192x128" in n for n in names(4608, 4096, 11008))  # three full rounds, the loop's two with 32 tiles
+    assert all("192x128" in n for n in names(3000, 4096, 4096))  # no multiple of 256: the loop cannot take it
