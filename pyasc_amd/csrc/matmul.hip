@@ -123,12 +123,20 @@ const TileFn kTileF32[asc::tile::kNumF32] = ASC_TILE_TABLE_F32(asc_tile_f32_);
 // The tile launch that takes the call of a checked, non-empty MmLaunch, or T.index < 0 when
 // L's own kernel runs it: K == 0 (no operand may be read), the tile-aligned loop on its own
 // 256x256 tiles (4096^3 bf16: 114.8 us against 115.8), and fp32 in 16x16 blocks: up to 256 of them on
-// operands that are not 16-byte aligned (100x301x501: 6.6 us against 7.6), and short products.
+// operands that are not 16-byte aligned (100x301x501: 6.6 us against 7.6), and short products.  Nor do tiles
+// take a 16-bit product of up to 256 columns in place of A, or of up to 256 rows too in place of B: it
+// is right where one workgroup reads what it overwrites, as the 256x256 tiles' kernels do.
 void make_tile(int32_t in_dtype, int32_t out_dtype, const MmLaunch& L, TileLaunch& T) {
   T = TileLaunch{};
   const GemmArgs& g = L.p;
   if (g.K == 0) return;
-  const int es = in_dtype == ASC_DT_FLOAT32 ? 4 : 2;
+  const int es = in_dtype == ASC_DT_FLOAT32 ? 4 : 2, oes = out_dtype == ASC_DT_FLOAT32 ? 4 : 2;
+  const int64_t c_bytes = int64_t{g.N} * oes;
+  if (es == 2 && g.N <= BN && (asc::tile::in_place(g.a, g.lda * 2, int64_t{g.K} * 2, g.c, g.ldc * oes, c_bytes) ||
+                               (g.M <= BM && asc::tile::in_place(g.b, g.ldb * 2, int64_t{g.N} * 2, g.c, g.ldc * oes,
+                                                                 c_bytes)))) {
+    return;
+  }
   const bool dma = asc::tile::dma_takes(g.a, g.b, g.N, g.K, g.lda, g.ldb, es);
   if (in_dtype == ASC_DT_FLOAT32) {
     if (!dma && ((g.M + 15) / 16) * static_cast<int64_t>((g.N + 15) / 16) <= asc::tile::kCus) return;

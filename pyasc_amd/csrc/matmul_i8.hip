@@ -68,11 +68,17 @@ using TileFn = void (*)(asc::gemm::TileArgs);
 const TileFn kTileI8[asc::tile::kNumDma + asc::tile::kNumAny] = ASC_TILE_TABLE_MFMA(asc_tile_i8_);
 
 // The tile launch that takes the call of a checked, non-empty I8Launch, or T.index < 0 when
-// L's own kernel runs it: K == 0, or the tile-aligned loop on its own 256x256 tiles.
+// L's own kernel runs it: K == 0, a C in place of an operand (as in matmul.hip), or the tile-aligned
+// loop on its own 256x256 tiles.
 void make_tile(int mode, const I8Launch& L, TileLaunch& T) {
   T = TileLaunch{};
   const I8Args& g = L.p;
   if (g.K == 0) return;
+  const int64_t c_bytes = int64_t{g.N} * (mode == 1 ? 2 : 4);
+  if (g.N <= BN && (asc::tile::in_place(g.a, g.K, g.K, g.c, c_bytes, c_bytes) ||
+                    (g.M <= BM && asc::tile::in_place(g.b, g.N, g.N, g.c, c_bytes, c_bytes)))) {
+    return;
+  }
   const bool dma = asc::tile::dma_takes(g.a, g.b, g.N, g.K, g.K, g.N, 1);
   const bool fast = L.kernel < 2;
   asc::tile::choose_mfma(1, dma, fast, g.M, g.N, g.K, T);

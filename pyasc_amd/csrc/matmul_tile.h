@@ -186,6 +186,17 @@ inline void choose(const Variant* table, int first, int last, int64_t M, int64_t
   }
 }
 
+// Whether C lies in place of an operand: rows of `c_bytes` and `bytes`, both `pitch` bytes apart,
+// that start within one row of each other and share memory.
+inline bool in_place(const void* x, int64_t pitch, int64_t bytes, const void* c, int64_t c_pitch, int64_t c_bytes) {
+  if (pitch != c_pitch) return false;
+  const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), c0 = reinterpret_cast<uintptr_t>(c);
+  const int64_t shift = c0 >= x0 ? static_cast<int64_t>(c0 - x0) : -static_cast<int64_t>(x0 - c0);
+  if (shift <= -pitch || shift >= pitch) return false;
+  // C's row meets its own row of x, the next or the one before
+  return (shift < bytes && shift + c_bytes > 0) || shift + c_bytes > pitch || shift + pitch < bytes;
+}
+
 // Whether the direct-to-LDS variants can address the operands: 16-byte chunks throughout, and
 // offsets from a tile's first row or k-tile below the out-of-bounds mark of their 31 bits.
 inline bool dma_takes(const void* a, const void* b, int64_t N, int64_t K, int64_t lda, int64_t ldb, int es) {

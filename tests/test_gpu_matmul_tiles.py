@@ -138,3 +138,24 @@ def test_short_f32_products_take_blocks(device, shape):
     kernels.matmul(a, b, c, **kw)
     torch.cuda.synchronize()
     _check(c, a, b, bias, "leaky", 0.25)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("M,N", [(1000, 256), (300, 64), (513, 200), (1, 256)])
+def test_product_in_place_of_a(device, dtype, M, N):
+    # up to 256 columns: a workgroup of the 256x256 tiles' kernels reads whole rows before it writes them
+    g = torch.Generator(device=device).manual_seed(M + N)
+    a = torch.randn((M, N), generator=g, device=device).to(dtype)
+    b = (torch.randn((N, N), generator=g, device=device) / N ** 0.5).to(dtype)
+    x = a.clone()
+    assert "_tile_" not in kernels.matmul_dispatch(x, b, x).kernel.decode()
+    kernels.matmul(x, b, x)
+    torch.cuda.synchronize()
+    _check(x, a, b, None, "none", 0.0)
+    # A and C side by side in one buffer share no memory
+    buf = torch.full((M, 2 * N), 7.0, dtype=dtype, device=device)
+    buf[:, :N] = a
+    kernels.matmul(buf[:, :N], b, buf[:, N:])
+    torch.cuda.synchronize()
+    _check(buf[:, N:], a, b, None, "none", 0.0)
+    assert torch.equal(buf[:, :N], a)

@@ -156,3 +156,46 @@ def test_tile_aligned_products_keep_their_loop():
     assert all("192x128" in n for n in names(1536, 4096, 4096))  # one round of 192x128
     assert all("192x128" in n for n in names(4608, 4096, 11008))  # three full rounds, the loop's two with 32 tiles
     assert all("192x128" in n for n in names(3000, 4096, 4096))  # no multiple of 256: the loop cannot take it
+
+
+@settings(max_examples=1500, deadline=None)
+@given(in_dt=st.sampled_from([F32, F16, BF16]), out_dt=st.sampled_from([F32, F16, BF16]), M=st.integers(1, 12),
+       N=st.integers(1, 24), K=st.integers(1, 24), pad=st.integers(0, 40), shift=st.integers(-130, 130),
+       other=st.sampled_from("ab"))
+def test_products_in_place_keep_the_plans_kernel(in_dt, out_dt, M, N, K, pad, shift, other):
+    # C and an operand with one row pitch, C's rows moved by less than that: every byte of both, one
+    # by one.  Tiles take the product if and only if it shares none, or is fp32 (in 16x16 blocks or
+    # small tiles, of which one holds up to 16 columns as well).
+    es, oes = ES[in_dt], ES[out_dt]
+    pitch = (max(K * es, N * es, N * oes) + pad) // 4 * 4 + 4
+    at = A + shift % pitch // oes * oes * (1 if shift >= 0 else -1)
+    a, b = (A, 0x4000000) if other == "a" else (0x4000000, A)
+    lda, ldb = (pitch // es, N) if other == "a" else (K, pitch // es)
+    rows, cols = (M, K) if other == "a" else (K, N)
+    p = _native.LaunchPlan()
+    assert lib().asc_matmul_dispatch(in_dt, out_dt, a, b, at, 0, M, N, K, lda, ldb, pitch // oes, 0, 0.0,
+                                     ctypes.byref(p)) == 0
+    taken = {A + r * pitch + i for r in range(rows) for i in range(cols * es)}
+    shared = any(at + r * pitch + i in taken for r in range(M) for i in range(N * oes))
+    if in_dt != F32 and shared:
+        assert "_tile_" not in p.kernel.decode()
+    elif in_dt != F32 and M > 1 and rows > 1:  # (with a single row a neighbour's does not exist)
+        assert "_tile_" in p.kernel.decode()
+
+
+def test_in_place_beyond_one_workgroup_or_a_pitch_is_no_concern():
+    def tile(M, N, K, c, other_b=B, ldc=None):
+        p = _native.LaunchPlan()
+        assert lib().asc_matmul_dispatch(BF16, BF16, A, other_b, c, 0, M, N, K, K, N, ldc or N, 0, 0.0,
+                                         ctypes.byref(p)) == 0
+        return "_tile_" in p.kernel.decode()
+
+    assert not tile(1000, 256, 256, A) and tile(1000, 264, 264, A)  # more columns: never one workgroup's rows
+    assert not tile(256, 256, 256, B) and tile(257, 256, 257, B)    # in place of B: one workgroup
+    assert tile(1000, 64, 128, A)                                   # another pitch
+    assert not tile(1000, 64, 128, A, ldc=128) and tile(1000, 64, 64, A + 128, ldc=128)
+    for dequant, width in ((0, 4), (1, 2)):
+        for at, shared in ((A, True), (A + 256, False), (A - 64 * width, False), (A + 100, True)):
+            p = _native.LaunchPlan()
+            assert lib().asc_matmul_i8_dispatch(A, B, BIAS, at, 300, 64, 64 * width, dequant, 0, ctypes.byref(p)) == 0
+            assert ("_tile_" in p.kernel.decode()) == (not shared), (dequant, hex(at))
