@@ -109,10 +109,9 @@ int32_t make_launch(const void* q, const void* k, const void* v, void* o, float*
   p.scale_log2 = sm_scale * 1.4426950408889634f;
   p.causal = causal ? 1 : 0;
   L.head_dim = head_dim;
-  const int32_t rc = head_dim == 64 ? geometry<FaConfig<64>>(L) : geometry<FaConfig<128>>(L);
-  if (rc != ASC_OK || !dispatch || !prefers_split(L)) return rc;
-  L.split = true;
-  return head_dim == 64 ? geometry<FaSplit<64>>(L) : geometry<FaSplit<128>>(L);
+  L.split = dispatch && prefers_split(L);  // few workgroups: within every limit of the grid
+  if (L.split) return head_dim == 64 ? geometry<FaSplit<64>>(L) : geometry<FaSplit<128>>(L);
+  return head_dim == 64 ? geometry<FaConfig<64>>(L) : geometry<FaConfig<128>>(L);
 }
 
 int32_t fill_plan(const FaLaunch& L, asc_launch_plan_t* plan) {
