@@ -150,17 +150,17 @@ def load_library(path: Optional[Path] = None) -> ctypes.CDLL:
 _torch_c = None  # torch._C once the device is initialised and it has the calls used below
 
 
-def current_stream_handle() -> int:
-    """hipStream_t of torch's current stream on the current device, read without building
-    a torch Stream object (the launch paths ask for it on every call)."""
+def current_stream_handle(device: Optional[int] = None) -> int:
+    """hipStream_t of torch's current stream on the current (or the given) device, read without
+    building a torch Stream object (the launch paths ask for it on every call)."""
     global _torch_c
     c = _torch_c
     if c is not None and not c._cuda_isInBadFork():
-        return c._cuda_getCurrentRawStream(c._cuda_getDevice())
+        return c._cuda_getCurrentRawStream(c._cuda_getDevice() if device is None else device)
     import torch
     if getattr(torch._C, "_cuda_getCurrentRawStream", None) is None:
-        return int(torch.cuda.current_stream().cuda_stream)
-    handle = int(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+        return int(torch.cuda.current_stream(device).cuda_stream)
+    handle = int(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device is None else device))
     if hasattr(torch._C, "_cuda_getDevice") and hasattr(torch._C, "_cuda_isInBadFork"):
         _torch_c = torch._C
     return handle

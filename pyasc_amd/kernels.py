@@ -40,27 +40,20 @@ def _device_tensor(t: Any, name: str) -> torch.Tensor:
     return t
 
 
+def _stream_of(handle: int, device: torch.device) -> Any:
+    """Stream ``handle`` as torch's.  0 is the default stream, which an ExternalStream cannot name."""
+    return torch.cuda.ExternalStream(handle, device=device) if handle else torch.cuda.default_stream(device)
+
+
 def workspace_on(handle: int, numel: int, dtype: torch.dtype, device: torch.device) -> torch.Tensor:
     """A workspace for the launches of one call on stream ``handle``, freed when the call returns.
     It comes from that stream's pool of torch's allocator: a block of another stream's pool may
     still be in use by work queued there, and would be handed out again before the launches have
     run, while a block of the launch stream's pool is ordered with them on both sides."""
-    if handle == torch.cuda.current_stream(device).cuda_stream:
+    if handle == _native.current_stream_handle(device.index):
         return torch.empty(numel, dtype=dtype, device=device)
-    # handle 0 is the default stream, which an ExternalStream cannot name
-    stream = torch.cuda.ExternalStream(handle, device=device) if handle else torch.cuda.default_stream(device)
-    with torch.cuda.stream(stream):
+    with torch.cuda.stream(_stream_of(handle, device)):
         return torch.empty(numel, dtype=dtype, device=device)
-
-
-def _capturing(handle: int, device: torch.device) -> bool:
-    """Whether stream ``handle`` is recording a graph."""
-    if handle == torch.cuda.current_stream(device).cuda_stream:
-        return torch.cuda.is_current_stream_capturing()
-    if handle == 0:
-        return False  # the default stream cannot be captured
-    with torch.cuda.stream(torch.cuda.ExternalStream(handle, device=device)):
-        return torch.cuda.is_current_stream_capturing()
 
 
 def _held_by_a_graph(t: torch.Tensor) -> bool:
@@ -318,9 +311,9 @@ _REDUCE_SPLIT_MIN = 1 << 18
 
 def _reduce(x: torch.Tensor, out: torch.Tensor, op: str, rows: int, cols: int, dim: int, count: int, stream) -> None:
     """One reduction; one with few results over many elements gets a workspace (at most 64 KiB)
-    for its partial results, from the launch stream's pool of torch's allocator.  Under a capture
-    that torch does not know of, whose replays would find that workspace given to others, it
-    runs without one."""
+    for its partial results, from the launch stream's pool of torch's allocator as workspace_on's.
+    Under a capture that torch does not know of, whose replays would find that workspace given
+    to others, it runs without one."""
     handle = _stream(stream)
     args = (REDUCE_OPS[op], x.data_ptr(), out.data_ptr(), rows, cols, dim, count)
     nbytes = 0
@@ -329,11 +322,17 @@ def _reduce(x: torch.Tensor, out: torch.Tensor, op: str, rows: int, cols: int, d
     if nbytes == 0:
         _native.call("asc_reduce_f32", *args, handle)
         return
-    workspace = workspace_on(handle, nbytes, torch.uint8, x.device)
-    if _capturing(handle, x.device) and not _held_by_a_graph(workspace):
+    if handle == _native.current_stream_handle(x.device.index):
+        workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+        usable = not torch.cuda.is_current_stream_capturing() or _held_by_a_graph(workspace)
+    else:
+        with torch.cuda.stream(_stream_of(handle, x.device)):
+            workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+            usable = not torch.cuda.is_current_stream_capturing() or _held_by_a_graph(workspace)
+    if usable:
+        _native.call("asc_reduce_f32_ws", *args, workspace.data_ptr(), nbytes, handle)
+    else:
         _native.call("asc_reduce_f32", *args, handle)
-        return
-    _native.call("asc_reduce_f32_ws", *args, workspace.data_ptr(), nbytes, handle)
 
 
 def rms_norm(x: torch.Tensor, gamma: torch.Tensor, out: torch.Tensor, num_rows: int, num_cols: int,

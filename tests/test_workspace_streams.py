@@ -26,8 +26,6 @@ def streams(monkeypatch):
         yield
         state.current.pop()
 
-    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: SimpleNamespace(
-        cuda_stream=state.current[-1]))
     monkeypatch.setattr(torch.cuda, "default_stream", lambda device=None: SimpleNamespace(cuda_stream=0))
     # as torch's: a null pointer is no external stream but asks for one of the pool's
     monkeypatch.setattr(torch.cuda, "ExternalStream", lambda ptr, device=None: SimpleNamespace(
@@ -35,7 +33,7 @@ def streams(monkeypatch):
     monkeypatch.setattr(torch.cuda, "stream", use)
     state.capturing = set()
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state.current[-1] in state.capturing)
-    monkeypatch.setattr(_native, "current_stream_handle", lambda: state.current[-1])
+    monkeypatch.setattr(_native, "current_stream_handle", lambda device=None: state.current[-1])
     real_empty = torch.empty
 
     def empty(*args, **kwargs):
