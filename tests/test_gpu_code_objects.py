@@ -135,6 +135,9 @@ def _softmax_fused(**options):
     return softmax_kernel
 
 
+SOFTMAX_SEEN = set()
+
+
 def _softmax_inputs(dtype, rows, cols, seed, device, offset=0):
     g = torch.Generator().manual_seed(seed)
     base = (torch.randn(rows * cols + offset, generator=g) * 4).to(dtype).to(device)
@@ -144,20 +147,22 @@ def _softmax_inputs(dtype, rows, cols, seed, device, offset=0):
 
 
 @pytest.mark.parametrize("dtype,rows,cols,tile,offset", [
-    # one case per planned kernel: wave_1x2, wave_2x2, block_2x128 / 2x256 / 2x512 / 8x256, long
+    # one case per launched kernel: wave_1x2, wave_2x2, block_2x128 / 2x256 / 2x512 / 8x256, long, short_f32, wide_f32
     (torch.float32, 37, 100, 100, 0), (torch.float32, 64, 300, 300, 0), (torch.float32, 33, 1000, 1000, 0),
     (torch.float32, 16, 2000, 2000, 0), (torch.float32, 9, 4000, 4000, 0), (torch.float32, 5, 8000, 8000, 0),
-    (torch.float32, 3, 9000, 9000, 0),
+    (torch.float32, 3, 9000, 9000, 0), (torch.float32, 1030, 200, 200, 0), (torch.float32, 3, 20000, 20000, 0),
     (torch.float32, 64, 1024, 1000, 0),   # tile narrower than the row: the rest is untouched
     (torch.float32, 64, 1024, 1024, 1),   # unaligned rows
     (torch.float32, 30, 100, 128, 0),     # tile wider than the row: padded_f32
     (torch.float16, 64, 1024, 1024, 0), (torch.float16, 10, 100, 100, 1),  # f16
+    (torch.float16, 2000, 1024, 1024, 0), (torch.float16, 3, 20000, 20000, 0),  # f16, wide_f16
     (torch.float16, 30, 100, 128, 0),     # padded_f16
 ])
 def test_softmax_code_object_matches_library(device, cache_dir, dtype, rows, cols, tile, offset):
     x, out_co = _softmax_inputs(dtype, rows, cols, rows * cols + tile, device, offset)
     out_lib = out_co.clone()
-    plan = kernels.softmax_plan(x, out_co, rows, cols, tile, 16, False)
+    plan = kernels.softmax_dispatch(x, out_co, rows, cols, tile, 16, False)
+    SOFTMAX_SEEN.add(plan.kernel.decode())
     _softmax_rows()[16](x, out_co, rows, cols, tile)
     kernels.softmax_rows(x, out_lib, rows, cols, tile, 16)
     torch.cuda.synchronize()
@@ -168,6 +173,11 @@ def test_softmax_code_object_matches_library(device, cache_dir, dtype, rows, col
     if tile <= cols:
         torch.testing.assert_close(out_co[:, :n].float(), torch.softmax(x[:, :n].float(), dim=1),
                                    rtol=1e-3 if dtype == torch.float16 else 1e-5, atol=1e-6)
+
+
+def test_every_softmax_kernel_was_compared(device):
+    from pyasc_amd.launchers import SOFTMAX_DISPATCH_FUNCTIONS
+    assert SOFTMAX_SEEN == set(SOFTMAX_DISPATCH_FUNCTIONS)
 
 
 @pytest.mark.parametrize("dtype,rows,cols,block_size", [(torch.float32, 64, 1024, 4), (torch.float32, 100, 300, 3),
@@ -325,13 +335,25 @@ def _both_paths(library_path, run):
     return first, second
 
 
-@pytest.mark.parametrize("form,dtype,m,k,n", [
-    ("mnblock", torch.float16, 480, 224, 1344), ("mnblock", torch.bfloat16, 512, 256, 512),
-    ("tiled", torch.float16, 64, 128, 256), ("fixpipe", torch.float32, 64, 128, 128),
-    ("fixpipe", torch.float16, 64, 128, 256), ("fixpipe", torch.bfloat16, 1024, 512, 768),
-    ("chained", torch.bfloat16, 64, 64, 64), ("chained", torch.float16, 256, 256, 256)])
-def test_matmul_code_object_matches_library(device, cache_dir, library_path, form, dtype, m, k, n):
+@pytest.mark.parametrize("form,dtype,m,k,n,kernel", [
+    ("mnblock", torch.float16, 480, 224, 1344, "tile_f16_"), ("mnblock", torch.bfloat16, 512, 256, 512, "tile_bf16_"),
+    ("tiled", torch.float16, 64, 128, 256, "tile_f16_"), ("fixpipe", torch.float32, 64, 128, 128, "f32_mfma_f16"),
+    ("fixpipe", torch.float32, 300, 513, 301, "tile_f32_"), ("fixpipe", torch.float16, 64, 128, 256, "tile_f16_"),
+    ("fixpipe", torch.bfloat16, 1024, 512, 768, "tile_bf16_"), ("chained", torch.bfloat16, 64, 64, 64, "tile_bf16_"),
+    ("chained", torch.float16, 256, 256, 256, "tile_f16_"),
+    # the loops on 256x256 tiles: tile-aligned from 129 tiles up, checked with K == 0
+    ("tiled", torch.float16, 4096, 64, 4096, "mfma_f16_fast_f32"),
+    ("fixpipe", torch.bfloat16, 4096, 96, 4096, "mfma_bf16_fast_f16"),
+    ("tiled", torch.bfloat16, 3072, 128, 4096, "mfma_bf16_fast_f32"),
+    ("fixpipe", torch.float16, 300, 0, 200, "mfma_f16_checked_f16"),
+    ("fixpipe", torch.float32, 3000, 0, 3000, "f32_fma_f16")])
+def test_matmul_code_object_matches_library(device, cache_dir, library_path, form, dtype, m, k, n, kernel):
     import test_gpu_reference_style as ref
+    if form in ("tiled", "fixpipe"):
+        ad, bd = torch.empty((m, k), dtype=dtype, device=device), torch.empty((k, n), dtype=dtype, device=device)
+        cd = torch.empty((m, n), dtype=torch.float16 if form == "fixpipe" else torch.float32, device=device)
+        name = kernels.matmul_dispatch(ad, bd, cd, relu=form == "fixpipe").kernel.decode()
+        assert name.startswith(f"asc2_mm_{kernel}"), name
     g = torch.Generator().manual_seed(m + k + n)
     a = ((torch.rand((m, k), generator=g) - .5) * 4).to(dtype).to(device)
     b = ((torch.rand((k, n), generator=g) - .5) * 4).to(dtype).to(device)
@@ -363,13 +385,16 @@ def test_matmul_code_object_matches_library(device, cache_dir, library_path, for
         torch.testing.assert_close(co.float(), expect, atol=1e-2, rtol=1e-2)
 
 
-@pytest.mark.parametrize("m,k,n", [(512, 256, 512), (100, 64, 300), (256, 4096, 256)])
-def test_int8_code_object_matches_library(device, cache_dir, library_path, m, k, n):
+@pytest.mark.parametrize("m,k,n,kernel", [(512, 256, 512, "tile_"), (100, 64, 300, "tile_"), (256, 4096, 256, "tile_"),
+                                          (4096, 128, 4096, "fast_i32"), (3072, 64, 3072, "fast_i32")])
+def test_int8_code_object_matches_library(device, cache_dir, library_path, m, k, n, kernel):
     import test_gpu_reference_style as ref
     g = torch.Generator().manual_seed(m * n + k)
     a = torch.randint(-127, 128, (m, k), dtype=torch.int8, generator=g).to(device)
     b = torch.randint(-127, 128, (k, n), dtype=torch.int8, generator=g).to(device)
     scale = (torch.rand(n, generator=g) * 0.009 + 0.001).to(device)
+    name = kernels.matmul_i8_dispatch(a, b, torch.empty((m, n), dtype=torch.int32, device=device)).kernel.decode()
+    assert name.startswith(f"asc2_i8_{kernel}"), name
 
     def run():
         acc = torch.zeros((m, n), dtype=torch.int32, device=device)
@@ -383,12 +408,15 @@ def test_int8_code_object_matches_library(device, cache_dir, library_path, m, k,
     assert torch.equal(acc_co.cpu(), (a.cpu().double() @ b.cpu().double()).to(torch.int32))
 
 
-@pytest.mark.parametrize("B,H,S,D,causal", [(2, 4, 512, 128, False), (2, 4, 512, 128, True), (1, 3, 300, 64, True),
-                                            (1, 8, 1024, 64, False)])
-def test_attention_code_object_matches_library(device, cache_dir, library_path, B, H, S, D, causal):
+@pytest.mark.parametrize("B,H,S,D,causal,split", [
+    (2, 4, 512, 128, False, True), (2, 4, 512, 128, True, True), (1, 3, 300, 64, True, True), (1, 8, 1024, 64, False, True),
+    (2, 64, 500, 128, True, False), (2, 64, 500, 64, False, False)])
+def test_attention_code_object_matches_library(device, cache_dir, library_path, B, H, S, D, causal, split):
     from test_gpu_attention import flash_attention_fwd_kernel
     g = torch.Generator().manual_seed(S + D)
     q, k, v = ((torch.randn(B, H, S, D, generator=g)).to(torch.bfloat16).to(device) for _ in range(3))
+    name = kernels.flash_attention_dispatch(q, k, v, torch.empty_like(q), 1 / D ** 0.5, causal).kernel.decode()
+    assert name == f"asc2_fa_fwd_d{D}{'_split' if split else ''}"
 
     def run():
         o = torch.empty_like(q)

@@ -5,8 +5,9 @@ draws add shapes around each kernel's fast-path conditions. For the GEMMs those 
 multiples of the 256 x 256 output tile and of the k-tile, the same plus or minus 1 or 31,
 tiny dimensions, and anything in between. For softmax they are the row lengths where the
 row body changes (256, 512, 1024, 2048, 4096, 8192 columns). A planner or bounds mistake
-that only one shape class shows fails here. Each test also checks that its draws reached
-every kernel they were meant to reach, using the launch plan's kernel name.
+that only one shape class shows fails here. Each GEMM draw runs through the entry, on the
+small tiles that the dispatch picks for shapes of this size, and its plan's kernel on
+256x256 tiles is launched from the code object as well; the tests check which kernels ran.
 
 Bars: int8 accumulators and dequant bit-exact; fp16/bf16 GEMM atol/rtol 1e-2 against the
 fp64-accumulated oracle; fp32 softmax rtol 1e-6, atol 0; attention atol/rtol 1e-2."""
@@ -15,7 +16,8 @@ import pytest
 import torch
 
 from oracle import asc2_oracle as O
-from pyasc_amd import kernels
+from pyasc_amd import kernels, launchers
+from pyasc_amd.asc.runtime import module
 
 pytestmark = pytest.mark.gpu
 
@@ -51,8 +53,23 @@ GEMM_SHAPES = _gemm_shapes(2026, 18, units=(256, 256, 32), tops=(768, 768, 1024)
 I8_SHAPES = _gemm_shapes(2027, 12, units=(256, 256, 64), tops=(768, 768, 512))
 
 
+@pytest.fixture(scope="module")
+def plan_kernels(device):
+    """The kernels of the matmul, int8 and softmax code objects, loaded from the prebuilt files."""
+    loaded = [module.load(co, str(co.path)) for co in (
+        launchers._matmul_code_object(None), launchers._i8_code_object(None), launchers.SOFTMAX_ROWS_CODE_OBJECT)]
+    yield {name: fn for lk in loaded for name, fn in lk.functions.items()}
+    for lk in loaded:
+        module.unload(lk)
+
+
+def _launch_plan(plan_kernels, plan):
+    module.launch_plan(plan_kernels, plan, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+
+
 def test_gemm_shapes_reach_both_loops():
-    # the draws hit the fast (tile-aligned, direct-to-LDS) and the checked loop alike
+    # the draws' plans name the fast (tile-aligned, direct-to-LDS) and the checked loop alike
     fast = [s for s in GEMM_SHAPES if s[0] % 256 == 0 and s[1] % 256 == 0 and s[2] % 32 == 0]
     assert 5 <= len(fast) <= len(GEMM_SHAPES) - 5
     fast8 = [s for s in I8_SHAPES if s[0] % 256 == 0 and s[1] % 256 == 0 and s[2] % 64 == 0]
@@ -60,7 +77,7 @@ def test_gemm_shapes_reach_both_loops():
 
 
 @pytest.mark.parametrize("idx", range(len(GEMM_SHAPES)))
-def test_matmul_random_shape(device, idx):
+def test_matmul_random_shape(device, plan_kernels, idx):
     M, N, K = GEMM_SHAPES[idx]
     rng = np.random.default_rng(idx)
     dtype = [torch.bfloat16, torch.float16][idx % 2]
@@ -70,17 +87,21 @@ def test_matmul_random_shape(device, idx):
     b = torch.randn(K, N, generator=g).to(dtype)
     c = torch.full((M, N), float(rng.integers(-9, 9)), dtype=out_dtype, device=device)
     ad, bd = a.to(device), b.to(device)
-    plan = kernels.matmul_plan(ad, bd, c).kernel.decode()
+    plan = kernels.matmul_plan(ad, bd, c)
     aligned = M % 256 == 0 and N % 256 == 0 and K % 32 == 0
-    assert ("_fast_" in plan) == aligned, (plan, M, N, K)
+    assert ("_fast_" if aligned else "_checked_") in plan.kernel.decode(), (plan.kernel, M, N, K)
+    assert "_tile_" in kernels.matmul_dispatch(ad, bd, c).kernel.decode()
     kernels.matmul(ad, bd, c)
     torch.cuda.synchronize()
     ref = torch.from_numpy(O.matmul(a.float().numpy(), b.float().numpy()))
     torch.testing.assert_close(c.cpu().float(), ref.to(out_dtype).float(), atol=1e-2, rtol=1e-2)
+    c.fill_(float(rng.integers(-9, 9)))
+    _launch_plan(plan_kernels, plan)
+    torch.testing.assert_close(c.cpu().float(), ref.to(out_dtype).float(), atol=1e-2, rtol=1e-2)
 
 
 @pytest.mark.parametrize("idx", range(len(I8_SHAPES)))
-def test_matmul_i8_random_shape(device, idx):
+def test_matmul_i8_random_shape(device, plan_kernels, idx):
     M, N, K = I8_SHAPES[idx]
     g = torch.Generator().manual_seed(2000 + idx)
     a = torch.randint(-127, 128, (M, K), dtype=torch.int8, generator=g)
@@ -89,16 +110,49 @@ def test_matmul_i8_random_shape(device, idx):
     ad, bd = a.to(device), b.to(device)
     acc = torch.full((M, N), -5, dtype=torch.int32, device=device)
     out = torch.full((M, N), 3.0, dtype=torch.float16, device=device)
-    plan = kernels.matmul_i8_plan(ad, bd, acc).kernel.decode()
+    scale_d = scale.to(device)
+    plans = kernels.matmul_i8_plan(ad, bd, acc), kernels.matmul_i8_plan(ad, bd, out, scale=scale_d)
     aligned = M % 256 == 0 and N % 256 == 0 and K % 64 == 0
-    assert ("_fast_" in plan) == aligned, (plan, M, N, K)
+    assert all(("_fast_" if aligned else "_checked_") in p.kernel.decode() for p in plans), (M, N, K)
+    assert "_tile_" in kernels.matmul_i8_dispatch(ad, bd, acc).kernel.decode()
     kernels.matmul_i8(ad, bd, acc)
-    kernels.matmul_i8(ad, bd, out, scale=scale.to(device))
+    kernels.matmul_i8(ad, bd, out, scale=scale_d)
     torch.cuda.synchronize()
     expect = O.matmul_i8_acc(a.numpy(), b.numpy())
-    np.testing.assert_array_equal(acc.cpu().numpy(), expect)
-    np.testing.assert_array_equal(out.cpu().numpy().view(np.uint16),
-                                  O.dequant_f16(expect, scale.numpy()).view(np.uint16))
+
+    def check():
+        np.testing.assert_array_equal(acc.cpu().numpy(), expect)
+        np.testing.assert_array_equal(out.cpu().numpy().view(np.uint16),
+                                      O.dequant_f16(expect, scale.numpy()).view(np.uint16))
+
+    check()
+    acc.fill_(-5)
+    out.fill_(3.0)
+    for p in plans:
+        _launch_plan(plan_kernels, p)
+    check()
+
+
+@pytest.mark.parametrize("dtype,M,N,K", [(t, M, N, K) for t in (torch.bfloat16, torch.float16, torch.int8)
+                                         for M, N, K in ((4096, 4096, 96), (3072, 4096, 64))] +
+                         [(torch.bfloat16, 768, 512, 0), (torch.float16, 700, 500, 0)])
+def test_entries_on_256x256_tiles(device, dtype, M, N, K):
+    # what the entries themselves still run on those tiles: enough of them, and K == 0
+    g = torch.Generator(device=device).manual_seed(M + K)
+    if dtype == torch.int8:
+        K = K // 64 * 64
+        a, b = (torch.randint(-127, 128, s, generator=g, device=device, dtype=dtype) for s in ((M, K), (K, N)))
+        c = torch.full((M, N), 7, dtype=torch.int32, device=device)
+        name, run = kernels.matmul_i8_dispatch(a, b, c).kernel.decode(), kernels.matmul_i8
+    else:
+        a, b = (torch.randn(s, generator=g, device=device).to(dtype) for s in ((M, K), (K, N)))
+        c = torch.full((M, N), 7.0, device=device)
+        name, run = kernels.matmul_dispatch(a, b, c).kernel.decode(), kernels.matmul
+    assert ("_fast_" if K else "_checked_") in name, name
+    run(a, b, c)
+    torch.cuda.synchronize()
+    exact, bound = a.double() @ b.double(), K * 2.0 ** -23 * (a.double().abs() @ b.double().abs())
+    assert ((c.double() - exact).abs() <= (0 if dtype == torch.int8 else bound)).all()
 
 
 def _softmax_draws(seed: int, n: int):
@@ -113,7 +167,9 @@ def _softmax_draws(seed: int, n: int):
     return draws
 
 
-SOFTMAX_DRAWS = _softmax_draws(2030, 18)  # a seed whose draws reach all eight fp32 bodies
+SOFTMAX_DRAWS = _softmax_draws(2030, 18)  # a seed whose draws' plans reach all eight fp32 bodies
+# what only the dispatch names: many short rows, and rows past 16384 columns
+SOFTMAX_DRAWS += [(1025, 64, 0), (2000, 333, 0), (3, 16385, 0), (2, 50001, 0)]
 
 
 @pytest.mark.parametrize("idx", range(len(SOFTMAX_DRAWS)))
@@ -129,14 +185,34 @@ def test_softmax_random_shape(device, idx):
 
 
 def test_softmax_draws_reach_every_row_body(device):
-    # the row-length draws, and the padded form, cover each fp32 softmax kernel
-    seen = set()
+    # the row-length draws, and the padded form, cover each fp32 softmax kernel that an entry launches
+    plans, launched = set(), set()
     for rows, cols, pad in SOFTMAX_DRAWS:
         x = torch.empty(rows, cols, device=device)
-        seen.add(kernels.softmax_plan(x, x, rows, cols, cols + pad, 16, False).kernel.decode())
+        args = (x, x, rows, cols, cols + pad, 16, False)
+        plans.add(kernels.softmax_plan(*args).kernel.decode())
+        launched.add(kernels.softmax_dispatch(*args).kernel.decode())
     body = {"wave_1x2", "wave_2x2", "block_2x128", "block_2x256", "block_2x512", "block_8x256", "long",
             "padded_f32"}
-    assert {s.split("asc2_softmax_")[-1] for s in seen} == body
+    assert {s.split("asc2_softmax_")[-1] for s in plans} == body
+    assert {s.split("asc2_softmax_")[-1] for s in launched} == body | {"short_f32", "wide_f32"}
+
+
+@pytest.mark.parametrize("dtype,cols", [(torch.float32, 16385), (torch.float32, 50001), (torch.float16, 16378),
+                                        (torch.float16, 70001)])
+def test_plans_of_long_rows(device, plan_kernels, dtype, cols):
+    # 256 threads per row, in two passes: what the entries launch for more than 2^22 such rows
+    x = (torch.randn(6, cols, generator=torch.Generator().manual_seed(cols)) * 2).to(dtype)
+    xd, out = x.to(device), torch.full((6, cols), 9.0, dtype=dtype, device=device)
+    plan = kernels.softmax_plan(xd, out, 6, cols, cols, 16, False)
+    assert plan.kernel.decode() == f"asc2_softmax_{'long' if dtype == torch.float32 else 'f16'}"
+    module.launch(plan_kernels[plan.kernel.decode()], plan.grid, plan.block,
+                  [("ptr", xd.data_ptr()), ("ptr", out.data_ptr()), ("i64", plan.rows), ("i64", plan.stride),
+                   ("i32", plan.len), ("i32", plan.flag)], torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    ref = torch.softmax(x.double(), dim=1)
+    tol = dict(rtol=2.0 ** -10, atol=2.0 ** -24) if dtype == torch.float16 else dict(rtol=2e-6, atol=0)
+    torch.testing.assert_close(out.cpu().double(), ref, **tol)
 
 
 def _attention_draws(seed: int, n: int):

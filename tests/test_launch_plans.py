@@ -1,8 +1,9 @@
 """asc_matmul_plan, asc_matmul_i8_plan, asc_flash_attention_plan (and, over random shapes,
-asc_softmax_plan) without a GPU: the launch each library entry point makes, as a
-code-object kernel name, grid, block and the kernel's argument struct as a blob.  The asc2 code-object path replays these plans; the GPU
-tests compare its results with the library's bit for bit.  Here: the kernel choice, the
-blob's fields, and that a plan fails exactly where its entry point does."""
+asc_softmax_plan) without a GPU: a launch of each entry point's work by its general kernel, as a
+code-object kernel name, grid, block and the kernel's argument struct as a blob.  The launch
+that the entries themselves make, and the asc2 code-object path replays, is the dispatch
+entries'; a plan is that launch where its kernel is the fastest.  Here: the choice among the
+general kernels, the blob's fields, and that a plan fails exactly where its entry point does."""
 import ctypes
 import math
 import struct

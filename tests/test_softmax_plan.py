@@ -1,6 +1,7 @@
-"""asc_softmax_plan without a GPU: the launch the softmax entries make (kernel, grid, block,
-arguments), which the asc2 code-object path replays through asc_module_launch.  The kernel
-choice at every row-length boundary, the coverage arguments of both reference kernels
+"""asc_softmax_plan without a GPU: a launch of the softmax entries' rows (kernel, grid, block,
+arguments) by a kernel chosen by type and row length alone; the launch that the entries make is
+asc_softmax_dispatch's, which may take another by the number of rows.  The kernel choice at
+every row-length boundary, the coverage arguments of both reference kernels
 (python/test/asc2/kernels/test_softmax.py:16-27, test_softmax_fused.py:16-24), the
 alignment flag, and the entries' own argument errors."""
 import ctypes
