@@ -212,8 +212,8 @@ int32_t asc_softmax_blocks_f16(const void* x, void* out, int64_t num_rows,
                                int64_t num_cols, int32_t block_size,
                                int32_t grid, asc_stream_t stream);
 
-/* A launch of the four softmax entries above, chosen by dtype and row length, for
- * a launcher that runs the kernels from the code object
+/* A launch of the four softmax entries above, chosen by dtype and row length (not
+ * always the one they make: asc_softmax_dispatch below), for a launcher that runs the kernels from the code object
  * pyasc_amd/lib/co/asc2_softmax.hsaco through asc_module_launch.  No counterpart in the
  * reference, whose compiler fixes the launch inside the kernel binary.
  * dtype ASC_DT_FLOAT32 / FLOAT16; fused 0 for asc_softmax_rows_* (size is
@@ -230,7 +230,8 @@ typedef struct asc_softmax_plan {
   int64_t rows;
   int64_t stride;
   int32_t len;
-  int32_t flag;
+  int32_t flag; /* padded tiles: tile_size - num_cols; else whether rows start on
+                   16-byte addresses (float32) or are whole 16-byte vectors (float16) */
 } asc_softmax_plan_t;
 int32_t asc_softmax_plan(int32_t dtype, int32_t fused, const void* x,
                          const void* out, int64_t num_rows, int64_t num_cols,
@@ -263,7 +264,7 @@ int32_t asc_reduce_f32(int32_t op, const float* x, float* out, int64_t rows,
  * be used).
  * The workspace (NULL: as asc_reduce_f32) must be 4-byte aligned, hold that many
  * bytes and not overlap x or out; both launches run in order on `stream`, so it
- * may be reused once they have run. */
+ * may be reused once they have run, and a captured call needs it at every replay. */
 int32_t asc_reduce_f32_workspace(int64_t rows, int64_t cols, int32_t dim);
 int32_t asc_reduce_f32_ws(int32_t op, const float* x, float* out, int64_t rows,
                           int64_t cols, int32_t dim, int64_t out_count,
@@ -359,8 +360,9 @@ int32_t asc_matmul_plan(int32_t in_dtype, int32_t out_dtype, const void* a,
                         asc_launch_plan_t* plan);
 /* The launch asc_matmul_bias_act makes with these arguments (asc_matmul(...,
  * relu) is act = relu, bias NULL): asc_matmul_plan's where its kernel is the
- * fastest for the shape, else one of the tile kernels asc2_mm_tile_* of the same
- * code object.  Same arguments, checks and errors as asc_matmul_plan. */
+ * fastest for the shape, where K is 0 or where C lies in place of A or B, else one
+ * of the tile kernels asc2_mm_tile_* of the same code object.  Same arguments,
+ * checks and errors as asc_matmul_plan. */
 int32_t asc_matmul_dispatch(int32_t in_dtype, int32_t out_dtype, const void* a,
                             const void* b, void* c, const float* bias,
                             int64_t M, int64_t N, int64_t K, int64_t lda,

@@ -690,8 +690,8 @@ __device__ __forceinline__ void fa_fwd_body(const FaArgs& p) {
 // Bound by the chain of tiles each wave goes through (about 0.8 us a tile at head_dim 64, 1.5 at
 // 128, one wave per SIMD): the chain is a quarter of the sequence, and four (head_dim 64) or eight
 // times as many workgroups as fa_fwd_body's spread over the CUs.  In exchange K and V are read
-// once per 32 queries.  fa_fwd_body, here (us, non-causal): 2x8 heads, 777 keys, head_dim 64: 13.8,
-// 10.2; 8 heads, 1024 keys, head_dim 128: 27.6, 12.6; 1 head, 4096 keys: 86.5, 28.9.
+// once per 32 queries.  fa_fwd_body, here (us, non-causal): 2x8 heads, 777 keys, head_dim 64: 13.0,
+// 9.4; 8 heads, 1024 keys, head_dim 128: 26.4, 11.6; 1 head, 4096 keys: 84.0, 26.7.
 // (Two query blocks per wave, QB = 2, halve the reads but double the chain's MFMAs: 18.8 us for
 // the 8 heads, and at most 15% faster where the launch fills the chip twice, where
 // fa_fwd_body is the better one in most cases.)

@@ -262,7 +262,7 @@ struct TileGemm {
     for (int i = 0; i < kLoadsB; ++i) *reinterpret_cast<u32x4*>(base + kBOff + (gw * kLoadsB + i) * 1024) = r.b[i];
   }
 
-  // ---- operands of k-step `step` (0, 1) from stage kS
+  // ---- operands of k-step `step` (0 .. kSteps - 1) from stage kS
   __device__ __forceinline__ static int b_off(int row, int col) {
     const int byte = col * kES;
     return row * kRowBytes + (((byte >> 4) ^ b_swz(row)) << 4) + (byte & 15);

@@ -9,7 +9,8 @@
 //   dim 1: a wave per row, or a workgroup per row when there are few long rows; 16-byte
 //          loads at element alignment, in-lane accumulation, DPP/permlane combine
 //          (HBM-bound: 4 B per element).
-//   dim 0: a workgroup per 64 columns walks the rows, 64 at a time, 16 bytes per lane.
+//   dim 0: a workgroup per 64 columns walks the rows, 64 at a time, 16 bytes per lane; a
+//          thread per four columns where rows are few or columns very many.
 //   all:   one 1024-thread block.
 // Few results leave most CUs idle: asc_reduce_f32_ws, with a workspace, splits the rows (dim
 // 0) or the elements (all) over enough workgroups to fill the chip, and a second launch
@@ -26,7 +27,6 @@
 
 #include "common.h"
 #include "numeric.h"
-#include "rows.h"
 
 namespace {
 
